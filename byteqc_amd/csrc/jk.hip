@@ -418,6 +418,7 @@ static std::vector<std::pair<long long, int>> g_ck_override;  // (key, ck)
 // flushes of the lane accumulators; 4-6 % over 64), the spilling 108-component
 // classes with 32-64 and the wave kernels with 64; for batches of small
 // molecules (4-40 H2O def2-SVP, at most ~1000 AOs) with 32, 16 and 16.
+// Launches with little work use shorter items (item_tile).
 #define BQC_TILE_BIG_NAO 2048
 #define BQC_TILE_HUGE_NAO 8192
 static bool g_ck_all_set[2] = {false, false};  // a tile set for all classes of a kind
@@ -427,11 +428,13 @@ static int class_components(int cls) {
     return nc(cls / 1000) * nc(cls / 100 % 10) * nc(cls / 10 % 10) * nc(cls % 10);
 }
 
-static int tile_for(int kind, int cls, int prec, int nao) {
+static int tile_for(int kind, int cls, int prec, int nao, bool *fixed = nullptr) {
     long long key = ((long long)kind * 10000 + cls) * 2 + prec;
+    if (fixed) *fixed = true;
     for (auto &kv : g_ck_override)
         if (kv.first == key) return kv.second;
     if (g_ck_all_set[kind == 1 ? 0 : 1]) return kind == 1 ? g_ck_rows : g_ck_wave;
+    if (fixed) *fixed = false;
     // three size bands, read off the autotuner on MI355X (batches of 4-40
     // waters, 64 waters cc-pVDZ, 128 waters cc-pVTZ): longer Q ranges per
     // item pay as the molecule grows
@@ -569,17 +572,12 @@ static void side_order(const int *bins, int nbins, const int *order, int npairs_
     }
 }
 
-// Adds one task to the plan.  Each precision takes the row kernel of the
-// class when there is one within the scratch and LDS limits, else the wave
-// kernel.  Returns -1 if a precision has neither (the generic kernels take
-// the task).
-template <template <class> class V>
-static int plan_task(BuildPlanT<V> &bp_, const TaskCtx &c, const int *bra_order,
-                     const JKArgs &jk, const PairData &pd) {
-    if (!bra_order || c.gen) return -1;
-    RowKernel k[2];
-    int wv[2];
-    bool fp32 = true;
+// Kernels of a task per precision: the row kernel of the class when there is
+// one within the scratch and LDS limits, else the wave kernel.  False if a
+// precision has neither (the generic kernels take the task).  *log_cut: the
+// precision rule with a row class that has no FP32 instance kept in FP64.
+static bool pick_kernels(const TaskCtx &c, RowKernel (&k)[2], int (&wv)[2], double *log_cut) {
+    *log_cut = c.log_cut;
     for (int prec = 0; prec < 2; ++prec) {
         RowKernel r = c.swap ? g_rows[0][prec][c.pkl][c.pij] : g_rows[0][prec][c.pij][c.pkl];
         RowKernel w = c.swap ? g_waves[prec][c.pkl][c.pij] : g_waves[prec][c.pij][c.pkl];
@@ -592,13 +590,101 @@ static int plan_task(BuildPlanT<V> &bp_, const TaskCtx &c, const int *bra_order,
         } else if (prec == 1 && !wv[0]) {
             k[1] = k[0];
             wv[1] = 0;
-            fp32 = false;
+            *log_cut = -1e300;
         } else {
-            return -1;
+            return false;
         }
     }
-    // a row class without an FP32 instance runs all its quartets in FP64
-    const double log_cut = fp32 ? c.log_cut : -1e300;
+    return true;
+}
+
+// First Q bin of P bin s whose quartets run in FP32 (nbins - s if none).
+static int fp32_split(const TaskCtx &c, int cp_p, int cp_q, const int *pbins, const int *qbins,
+                      int s, double log_cut) {
+    const double ubp = bin_ub(c, cp_p, pbins, s);
+    for (int bq = 0; bq < c.nbins - s; ++bq)
+        if (ubp + bin_ub(c, cp_q, qbins, bq) < log_cut) return bq;
+    return c.nbins - s;
+}
+
+// Work of the launches of a build, one entry per evaluated class and
+// precision, in primitive-quartet steps of a wavefront.  A step of a task
+// costs its primitive quartets plus BQC_STEP_BASE for the digestion.
+#define BQC_STEP_BASE 2
+struct ClassLoad {
+    double cost[2][BQC_NPAIRID][BQC_NPAIRID];
+    ClassLoad() { memset(cost, 0, sizeof(cost)); }
+    double &at(const TaskCtx &c, int prec) {
+        return c.swap ? cost[prec][c.pkl][c.pij] : cost[prec][c.pij][c.pkl];
+    }
+};
+
+static int step_cost(const TaskCtx &c) {
+    return c.bp->cptype[c.cp_ij].nprim_12 * c.bp->cptype[c.cp_kl].nprim_12 + BQC_STEP_BASE;
+}
+
+static void add_load(ClassLoad &load, const TaskCtx &c) {
+    RowKernel k[2];
+    int wv[2];
+    double log_cut;
+    if (c.gen || !pick_kernels(c, k, wv, &log_cut)) return;
+    const int *pbins = c.swap ? c.bins_kl : c.bins_ij, *qbins = c.swap ? c.bins_ij : c.bins_kl;
+    const int cp_p = c.swap ? c.cp_kl : c.cp_ij, cp_q = c.swap ? c.cp_ij : c.cp_kl;
+    double steps[2] = {0, 0};
+    for (int s = 0; s < c.nbins; ++s) {
+        const int np = pbins[s + 1] - pbins[s];
+        if (np <= 0) continue;
+        const int qmax = qbins[c.nbins - s];
+        const int qsplit = qbins[fp32_split(c, cp_p, cp_q, pbins, qbins, s, log_cut)];
+        steps[0] += (wv[0] ? np : np / 64.0) * qsplit;
+        steps[1] += (wv[1] ? np : np / 64.0) * (qmax - qsplit);
+    }
+    for (int prec = 0; prec < 2; ++prec) load.at(c, prec) += steps[prec] * step_cost(c);
+}
+
+// Q pairs per work item of a task: at most the class's tile.  A wavefront
+// walks its Q range one step after the other, so the longest item bounds the
+// launch from below, and a launch with fewer items than the device holds
+// wavefronts leaves CUs idle.  Items therefore cost what BQC_FILL_HI items per
+// resident wavefront allow (so the items of a launch cost about the same
+// whatever their tasks' contraction), or BQC_ITEM_MIN where that would be
+// shorter (every item pays its lane set-up and accumulator flushes), but no
+// more than BQC_FILL_LO items per resident wavefront allow.  Measured on
+// MI355X against fixed tiles (ms): 1 water cc-pVDZ 7.5 -> 1.2, 8 waters
+// cc-pVDZ 16.8 -> 4.1, 40 waters def2-SVP mixed 204 -> 68, 5 waters cc-pVTZ
+// 63.6 -> 27.  BQC_FILL_HI 4 / 8 / 16: 266 / 255 / 251 for 12 molecules
+// def2-SVP, 200 / 201 / 205 for 24 waters cc-pVTZ; BQC_FILL_LO 0.06 / 0.25 /
+// 0.5: 32.8 / 27.0 / 26.7 for 5 waters cc-pVTZ, 4.6 / 4.1 / 4.8 for 8 waters
+// cc-pVDZ; BQC_ITEM_MIN 24 / 48 / 96 / 192: 12.6 / 11.8 / 11.8 / 13.8 for 13
+// waters cc-pVDZ with two densities.
+#define BQC_FILL_HI 8
+#define BQC_FILL_LO 0.25
+#define BQC_ITEM_MIN 96
+static int item_tile(ClassLoad &load, const TaskCtx &c, RowKernel kern, int wave, int prec,
+                     int nao) {
+    bool fixed;
+    const int cap = tile_for(wave ? 4 : 1, eval_cls(c), prec, nao, &fixed);
+    if (fixed) return cap;
+    const unsigned waves = wave ? resident_blocks((const void *)kern, 64)
+                                : 4 * resident_blocks((const void *)kern, 256);
+    if (!waves) return cap;
+    const double per_wave = load.at(c, prec) / waves;
+    const double cost = std::max(per_wave / BQC_FILL_HI,
+                                 std::min(per_wave / BQC_FILL_LO, (double)BQC_ITEM_MIN));
+    const double ck = cost / step_cost(c);
+    return ck >= cap ? cap : (ck > 1 ? (int)ck : 1);
+}
+
+// Adds one task to the plan; load holds the work of the whole launch set.
+// Returns -1 if the generic kernels take the task.
+template <template <class> class V>
+static int plan_task(BuildPlanT<V> &bp_, const TaskCtx &c, const int *bra_order,
+                     const JKArgs &jk, const PairData &pd, ClassLoad &load) {
+    if (!bra_order || c.gen) return -1;
+    RowKernel k[2];
+    int wv[2];
+    double log_cut;
+    if (!pick_kernels(c, k, wv, &log_cut)) return -1;
     // split row class: a-side and b-side passes (FP64 builds of the class only)
     RowKernel ks[2] = {nullptr, nullptr};
     const int *order2 = nullptr;
@@ -682,21 +768,14 @@ static int plan_task(BuildPlanT<V> &bp_, const TaskCtx &c, const int *bra_order,
     auto q_limits = [&](int p, int &qmax, int &qsplit) {
         int s = (int)(std::upper_bound(pbins + 1, pbins + nbins + 1, p) - (pbins + 1));
         qmax = qbins[nbins - s];
-        double ubp = bin_ub(c, cp_p, pbins, s);
-        int split = nbins - s;
-        for (int bq = 0; bq < nbins - s; ++bq)
-            if (ubp + bin_ub(c, cp_q, qbins, bq) < log_cut) {
-                split = bq;
-                break;
-            }
-        qsplit = qbins[split];
+        qsplit = qbins[fp32_split(c, cp_p, cp_q, pbins, qbins, s, log_cut)];
     };
     // When one precision runs rows of 64 P pairs, the split of a row's first
     // pair holds for every pair of the row in both precisions, so the two
     // precisions cover each pair's Q range exactly once.
     const bool by_row = !wv[0] || !wv[1];
     for (int prec = 0; prec < 2; ++prec) {
-        const int ck = tile_for(wv[prec] ? 4 : 1, cls, prec, jk.nao);
+        const int ck = item_tile(load, c, k[prec], wv[prec], prec, jk.nao);
         const int step = wv[prec] ? 1 : 64;
         V<int> &it = g[prec]->items;
         for (int p = 0; p < np; p += step) {
@@ -1006,7 +1085,8 @@ static int task_ctx(TaskCtx &c, const MolArgs &a, int t, int nbins, int precisio
 
 // Plans tasks list[0, n) into plan; generic-kernel tasks go to *deferred.
 static int plan_refs(BuildPlan &plan, const MolArgs *m, const TaskRef *list, size_t n,
-                     int nbins, int precision, double fp32_cut, std::vector<Deferred> *deferred) {
+                     int nbins, int precision, double fp32_cut, ClassLoad &load,
+                     std::vector<Deferred> *deferred) {
     for (size_t i = 0; i < n; ++i) {
         const MolArgs &a = m[list[i].im];
         TaskCtx c;
@@ -1014,7 +1094,7 @@ static int plan_refs(BuildPlan &plan, const MolArgs *m, const TaskRef *list, siz
         if (err) return err;
         JKArgs jk = {a.vj, a.vk, a.dm, a.nao, a.n_dm};
         PairData pd = make_pair_data(a.bp);
-        err = plan_task(plan, c, a.bra_order, jk, pd);
+        err = plan_task(plan, c, a.bra_order, jk, pd, load);
         if (err < 0) {
             deferred->push_back(Deferred{c, jk, pd});
             err = 0;
@@ -1030,8 +1110,15 @@ static int plan_refs(BuildPlan &plan, const MolArgs *m, const TaskRef *list, siz
 // Generic-kernel tasks are appended to deferred in list order.
 static int plan_list(BuildPlan &plan, const MolArgs *m, const TaskRef *list, size_t n,
                      int nbins, int precision, double fp32_cut, std::vector<Deferred> &deferred) {
+    ClassLoad load;
+    for (size_t i = 0; i < n; ++i) {
+        TaskCtx c;
+        const int err = task_ctx(c, m[list[i].im], list[i].t, nbins, precision, fp32_cut);
+        if (err) return err;
+        add_load(load, c);
+    }
     const int nth = plan_threads(n);
-    if (nth < 2) return plan_refs(plan, m, list, n, nbins, precision, fp32_cut, &deferred);
+    if (nth < 2) return plan_refs(plan, m, list, n, nbins, precision, fp32_cut, load, &deferred);
     const size_t bsz = std::max<size_t>(4, n / ((size_t)nth * 8));
     const size_t nblk = (n + bsz - 1) / bsz;
     std::vector<BuildPlan> part(nblk);
@@ -1047,7 +1134,7 @@ static int plan_list(BuildPlan &plan, const MolArgs *m, const TaskRef *list, siz
         for (size_t b; (b = next.fetch_add(1)) < nblk;) {
             const size_t t0 = b * bsz, t1 = std::min(n, t0 + bsz);
             part_err[b] = plan_refs(part[b], m, list + t0, t1 - t0, nbins, precision, fp32_cut,
-                                    &part_def[b]);
+                                    load, &part_def[b]);
         }
     };
     std::vector<std::thread> th;
@@ -1138,18 +1225,23 @@ static int plan_molecules(BuildPlanT<V> &plan, const MolArgs *m, int nmol, int n
         }
         return 0;
     }
+    ClassLoad load;
+    for (int im = 0; im < nmol; ++im)
+        for (int t = 0; t < m[im].ntask; ++t) {
+            TaskCtx c;
+            const int err = task_ctx(c, m[im], t, nbins, precision, fp32_cut);
+            if (err) return err;
+            add_load(load, c);
+        }
     for (int im = 0; im < nmol; ++im) {
         const MolArgs &a = m[im];
         JKArgs jk = {a.vj, a.vk, a.dm, a.nao, a.n_dm};
         PairData pd = make_pair_data(a.bp);
         for (int t = 0; t < a.ntask; ++t) {
-            const int *bi = a.task_bins + (size_t)t * 2 * (nbins + 1);
-            const int *bk = bi + nbins + 1;
             TaskCtx c;
-            int err = task_init(c, a.bp, bi, bk, nbins, a.task_cp[2 * t], a.task_cp[2 * t + 1],
-                                a.log_q, a.task_dmax ? a.task_dmax[t] : 0, fp32_cut, precision);
+            int err = task_ctx(c, a, t, nbins, precision, fp32_cut);
             if (err) return err;
-            err = plan_task(plan, c, a.bra_order, jk, pd);
+            err = plan_task(plan, c, a.bra_order, jk, pd, load);
             if (err < 0 && deferred) {
                 deferred->push_back(Deferred{c, jk, pd});
                 err = 0;
@@ -1247,7 +1339,9 @@ int GINTbuild_jk(BasisProdCache *bpcache, double *vj, double *vk, double *dm, in
                            ? shell_order(bpcache, 0, cp_ij_id, cp_kl_id)
                            : nullptr;
     BuildPlan plan;
-    err = plan_task(plan, c, order, jk, pd);
+    ClassLoad load;
+    add_load(load, c);
+    err = plan_task(plan, c, order, jk, pd, load);
     if (err < 0) err = launch_quartets(c, jk, pd, stream, plan.flops);
     else if (err == 0) err = stage_and_launch(plan, stream);
     g_last_flops[0] = plan.flops[0];
