@@ -428,13 +428,16 @@ __global__ void __launch_bounds__(64, (wave_min_waves<LA, LB, LC, LD>()))
 typedef RowKernel WaveKernel;
 typedef WaveKernel WaveKernelTable[2][BQC_NPAIRID][BQC_NPAIRID];
 
-// Classes digested with the wavefront-per-quartet kernel (LDS budget: up to
-// (fd|fd) and (ff|fd), whose ~80 KB leave room for two workgroups per CU;
-// the planner refuses a kernel above the device's per-workgroup LDS).
+// Classes digested with the wavefront-per-quartet kernel: all above the row
+// kernel's, up to (ff|ff), whose 128 KB of LDS fit one workgroup per CU (the
+// planner refuses a kernel above the device's per-workgroup LDS).  (ff|ff)
+// quartets are few, so the alternative of one lane per quartet left the chip
+// empty behind single lanes of 10 000 components: 30 quartets of 5 waters
+// cc-pVTZ took 11.4 ms (0.3 ms here), 660 of 24 waters 25.8 ms (1.6 ms).
 template <int LA, int LB, int LC, int LD>
 constexpr bool use_wave() {
     using C = Cls<LA, LB, LC, LD>;
-    return C::NF > 81 && (3 * C::NR * C::GSZ + C::NF) * 8 <= 80000;
+    return C::NF > 81 && (3 * C::NR * C::GSZ + C::NF) * 8 <= 130000;
 }
 
 template <int LA, int LB, int LC, int LD>
