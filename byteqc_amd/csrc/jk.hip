@@ -120,6 +120,14 @@ struct TaskCtx {
     double qflops;       // FLOPs of one quartet of this class
 };
 
+// FLOPs of a task's quartets.
+static double task_flops(const TaskCtx &c) {
+    double n = 0;
+    for (int b = 0; b < c.nbins; ++b)
+        n += count_rect(0, c.bins_ij[c.nbins - b], c.bins_kl[b], c.bins_kl[b + 1], c.diag);
+    return n * c.qflops;
+}
+
 // log q upper bound of bin b of pair type cp (first pair of the bin in the
 // q-descending plan order); +inf for an empty bin or without log q
 static double bin_ub(const TaskCtx &c, int cp, const int *bins, int b) {
@@ -893,48 +901,117 @@ __global__ void fill_qrec(const TaskDesc *tasks, int ntask) {
 }
 
 template <template <class> class V>
+static int launch_group(const BuildPlanT<V> &p, const StagedT<V> &st, char *dev, size_t gi,
+                        hipStream_t stream) {
+    const GroupT<V> &g = p.groups[gi];
+    int nitems = (int)g.items.size() / 4;
+    if (!nitems) return 0;
+    const int4 *items = (const int4 *)(dev + st.off_items[gi]);
+    unsigned nblk = g.wave ? (unsigned)nitems : (unsigned)((nitems + 3) / 4);
+    unsigned nthr = g.wave ? 64 : 256;
+    int *ticket = nullptr;
+    // persistent grids: 64 waters cc-pVDZ 143.0 -> 136.5 ms, 256 small
+    // def2-SVP molecules 5.06 -> 4.69 s per batch (with per-XCD counters)
+    if (!g.wave && (g_persistent == 2 || (g_persistent == 1 && g.nao_max >= BQC_TILE_BIG_NAO))) {
+        // as many workgroups as stay resident at once; they drain the list
+        const unsigned cap = resident_blocks((const void *)g.kern, (int)nthr);
+        if (cap > 0 && cap < nblk) {
+            nblk = cap;
+            ticket = (int *)(dev + st.off_tickets) + gi * BQC_TICKET_SLICES;
+        }
+    }
+    LaunchRec rec;
+    if (prof_on())
+        record_launch(rec, g.cls, (g.wave ? 4 : 1) + 2 * g.prec + 8 * g.role_b, g.flops, g.nquart,
+                      stream);
+    hipLaunchKernelGGL(g.kern, dim3(nblk), dim3(nthr), 0, stream, (const TaskDesc *)dev, items,
+                       nitems, ticket);
+    if (prof_on()) keep_launch(rec, stream);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+        fprintf(stderr, "bqcjk: kernel launch failed: %s\n", hipGetErrorString(e));
+        return 1;
+    }
+    return 0;
+}
+
+// Side streams that run the launches of one build next to each other, with
+// the events that order them after the build's copies and before whatever
+// follows it on its own stream.
+#define BQC_SIDE_STREAMS 3
+struct SideStreams {
+    hipStream_t s[BQC_SIDE_STREAMS] = {};
+    hipEvent_t fork = nullptr, join[BQC_SIDE_STREAMS] = {};
+    int dev = -1;  // device they belong to; -1 before the first use
+    // true if they can be used on the current device
+    bool ready() {
+        int d = 0;
+        if (hipGetDevice(&d) != hipSuccess) return false;
+        if (dev < 0) {
+            bool ok = hipEventCreateWithFlags(&fork, hipEventDisableTiming) == hipSuccess;
+            for (int i = 0; i < BQC_SIDE_STREAMS && ok; ++i)
+                ok = hipStreamCreateWithFlags(&s[i], hipStreamNonBlocking) == hipSuccess &&
+                     hipEventCreateWithFlags(&join[i], hipEventDisableTiming) == hipSuccess;
+            if (!ok) {
+                destroy();
+                return false;
+            }
+            dev = d;
+        }
+        return dev == d;
+    }
+    void destroy() {
+        for (int i = 0; i < BQC_SIDE_STREAMS; ++i) {
+            if (s[i]) (void)hipStreamDestroy(s[i]);
+            if (join[i]) (void)hipEventDestroy(join[i]);
+            s[i] = nullptr;
+            join[i] = nullptr;
+        }
+        if (fork) (void)hipEventDestroy(fork);
+        fork = nullptr;
+        dev = -1;
+    }
+};
+
+// Launches every group: one after the other on the stream, or (side != NULL)
+// spread over the stream and the side streams.  Per-launch timing keeps them
+// on one stream, where a launch's events bracket that launch alone.
+template <template <class> class V>
 static int launch_groups(const BuildPlanT<V> &p, const StagedT<V> &st, char *dev,
-                         hipStream_t stream) {
-    const TaskDesc *tasks = (const TaskDesc *)dev;
+                         hipStream_t stream, SideStreams *side = nullptr) {
     if (!p.tasks.empty() && p.qmax > 0) {
         const int nt = (int)p.tasks.size();
         hipLaunchKernelGGL(fill_qrec, dim3((p.qmax + 255) / 256, nt < 65535 ? nt : 65535),
-                           dim3(256), 0, stream, tasks, nt);
+                           dim3(256), 0, stream, (const TaskDesc *)dev, nt);
         if (hipGetLastError() != hipSuccess) return 1;
     }
-    for (size_t gi = 0; gi < p.groups.size(); ++gi) {
-        const GroupT<V> &g = p.groups[gi];
-        int nitems = (int)g.items.size() / 4;
-        if (!nitems) continue;
-        const int4 *items = (const int4 *)(dev + st.off_items[gi]);
-        unsigned nblk = g.wave ? (unsigned)nitems : (unsigned)((nitems + 3) / 4);
-        unsigned nthr = g.wave ? 64 : 256;
-        int *ticket = nullptr;
-        // persistent grids: 64 waters cc-pVDZ 143.0 -> 136.5 ms, 256 small
-        // def2-SVP molecules 5.06 -> 4.69 s per batch (with per-XCD counters)
-        if (!g.wave &&
-            (g_persistent == 2 || (g_persistent == 1 && g.nao_max >= BQC_TILE_BIG_NAO))) {
-            // as many workgroups as stay resident at once; they drain the list
-            const unsigned cap = resident_blocks((const void *)g.kern, (int)nthr);
-            if (cap > 0 && cap < nblk) {
-                nblk = cap;
-                ticket = (int *)(dev + st.off_tickets) + gi * BQC_TICKET_SLICES;
-            }
-        }
-        LaunchRec rec;
-        if (prof_on())
-            record_launch(rec, g.cls, (g.wave ? 4 : 1) + 2 * g.prec + 8 * g.role_b, g.flops,
-                          g.nquart, stream);
-        hipLaunchKernelGGL(g.kern, dim3(nblk), dim3(nthr), 0, stream, tasks, items, nitems,
-                           ticket);
-        if (prof_on()) keep_launch(rec, stream);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) {
-            fprintf(stderr, "bqcjk: kernel launch failed: %s\n", hipGetErrorString(e));
-            return 1;
-        }
+    const size_t ng = p.groups.size();
+    if (!side || prof_on() || ng < 2 || !side->ready()) {
+        for (size_t gi = 0; gi < ng; ++gi)
+            if (launch_group(p, st, dev, gi, stream)) return 1;
+        return 0;
     }
-    return 0;
+    // longest first, each to the stream with the least queued so far
+    std::vector<std::pair<double, size_t>> order(ng);
+    for (size_t gi = 0; gi < ng; ++gi)
+        order[gi] = {-(10 + 0.1 * class_components(p.groups[gi].cls) + p.groups[gi].flops / 4e6),
+                     gi};
+    std::sort(order.begin(), order.end());
+    double queued[BQC_SIDE_STREAMS + 1] = {};
+    if (hipEventRecord(side->fork, stream) != hipSuccess) return 1;
+    for (int i = 0; i < BQC_SIDE_STREAMS; ++i)
+        if (hipStreamWaitEvent(side->s[i], side->fork, 0) != hipSuccess) return 1;
+    int err = 0;
+    for (const auto &o : order) {
+        const int k = (int)(std::min_element(queued, queued + BQC_SIDE_STREAMS + 1) - queued);
+        queued[k] -= o.first;
+        err |= launch_group(p, st, dev, o.second, k ? side->s[k - 1] : stream);
+    }
+    for (int i = 0; i < BQC_SIDE_STREAMS; ++i)
+        if (hipEventRecord(side->join[i], side->s[i]) != hipSuccess ||
+            hipStreamWaitEvent(stream, side->join[i], 0) != hipSuccess)
+            err = 1;
+    return err;
 }
 
 // Device images of the work lists of direct (non-graph) builds: a ring of
@@ -958,6 +1035,7 @@ struct StageSlot {
 struct StreamStage {
     StageSlot slot[BQC_STAGE_SLOTS];
     int next = 0;
+    SideStreams side;
 };
 static std::mutex g_stage_mu;
 static std::map<hipStream_t, StreamStage> g_stages;
@@ -967,7 +1045,7 @@ static StreamStage &stage_for(hipStream_t stream) {
     return g_stages[stream];
 }
 
-static int stage_and_launch(BuildPlan &p, hipStream_t stream) {
+static int stage_and_launch(BuildPlan &p, hipStream_t stream, bool spread = false) {
     if (p.groups.empty()) return 0;
     Staged st = stage_layout(p);
     StreamStage &sst = stage_for(stream);
@@ -1006,7 +1084,7 @@ static int stage_and_launch(BuildPlan &p, hipStream_t stream) {
         return 1;
     hipEventRecord(ss.evt, stream);
     ss.pending = true;
-    return launch_groups(p, st, ss.dws, stream);
+    return launch_groups(p, st, ss.dws, stream, spread ? &sst.side : nullptr);
 }
 
 struct MolArgs {
@@ -1158,10 +1236,18 @@ static int check_build_args(const MolArgs *m, int nmol, int nbins, int precision
 }
 
 // Direct builds: tasks grouped by integral class (classes in order of first
-// appearance, tasks in order inside a class), and each class staged and
-// launched as soon as it is planned, so the device runs the first classes
-// while the host plans the rest instead of waiting for the whole plan
-// (64 waters cc-pVDZ: 5.4 ms of planning ahead of the first launch).
+// appearance, tasks in order inside a class).  Below BQC_SPREAD_FLOPS all
+// classes are planned into one work list (one copy, one fill_qrec) and their
+// launches spread over several streams: a launch ends with some 0.1-0.3 ms of
+// a few long items, and launches of small molecules are nothing but that, so
+// the next class fills the chip meanwhile (ms on MI355X, one stream -> four: 4
+// waters def2-SVP 7.1 -> 5.1, 8 waters cc-pVDZ 4.0 -> 2.9, 5 waters cc-pVTZ
+// 16.1 -> 9.3, 24 waters cc-pVTZ 177 -> 165, 12 molecules def2-SVP 255 -> 250,
+// 64 waters cc-pVDZ 120 -> 120).  Above, each class is staged and launched as
+// soon as it is planned, so the device runs the first classes while the host
+// plans the rest (128 waters cc-pVTZ, 4e13 FLOPs: a launch's end is below 1 %
+// of it, planning ahead of all launches would not be hidden).
+#define BQC_SPREAD_FLOPS 4e12
 static int build_by_class(const MolArgs *m, int nmol, int nbins, int precision, double fp32_cut,
                           hipStream_t stream, double flops[2]) {
     flops[0] = flops[1] = 0;
@@ -1170,11 +1256,13 @@ static int build_by_class(const MolArgs *m, int nmol, int nbins, int precision, 
     register_kernels();
     std::vector<int> keys;
     std::vector<std::vector<TaskRef>> by_cls;
+    double work = 0;
     for (int im = 0; im < nmol; ++im)
         for (int t = 0; t < m[im].ntask; ++t) {
             TaskCtx c;
             err = task_ctx(c, m[im], t, nbins, precision, fp32_cut);
             if (err) return err;
+            work += task_flops(c);
             const int key = eval_cls(c);
             size_t k = 0;
             while (k < keys.size() && keys[k] != key) ++k;
@@ -1184,13 +1272,19 @@ static int build_by_class(const MolArgs *m, int nmol, int nbins, int precision, 
             }
             by_cls[k].push_back(TaskRef{im, t});
         }
+    const bool spread = work < BQC_SPREAD_FLOPS;
+    if (spread && by_cls.size() > 1) {
+        for (size_t k = 1; k < by_cls.size(); ++k)
+            by_cls[0].insert(by_cls[0].end(), by_cls[k].begin(), by_cls[k].end());
+        by_cls.resize(1);
+    }
     for (const std::vector<TaskRef> &list : by_cls) {
         BuildPlan plan;
         std::vector<Deferred> def;
         err = plan_list(plan, m, list.data(), list.size(), nbins, precision, fp32_cut, def);
         for (Deferred &d : def)
             if (!err) err = launch_quartets(d.c, d.jk, d.pd, stream, plan.flops);
-        if (!err) err = stage_and_launch(plan, stream);
+        if (!err) err = stage_and_launch(plan, stream, spread);
         flops[0] += plan.flops[0];
         flops[1] += plan.flops[1];
         if (err) return err;
@@ -1437,7 +1531,8 @@ __global__ void zero_ints(int *p, int n) {
     if (i < n) p[i] = 0;
 }
 
-// A captured batch: its own device image and the instantiated graph.
+// A captured batch: its own device image and the instantiated graph, whose
+// launches are parallel branches (24 molecules def2-SVP 97 -> 91 ms a replay).
 struct BQCGraph {
     hipGraph_t graph;
     hipGraphExec_t exec;
@@ -1475,6 +1570,8 @@ void *BQCgraph_capture(int nmol, BasisProdCache **bps, double **vj, double **vk,
         }
     }
     hipStream_t cs = nullptr;
+    SideStreams side;
+    if (!err) (void)side.ready();
     if (!err && hipStreamCreateWithFlags(&cs, hipStreamNonBlocking) != hipSuccess) err = 1;
     if (!err && hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal) != hipSuccess) err = 1;
     if (!err) {
@@ -1488,7 +1585,7 @@ void *BQCgraph_capture(int nmol, BasisProdCache **bps, double **vj, double **vk,
             const int ng = (int)plan.groups.size() * BQC_TICKET_SLICES;
             hipLaunchKernelGGL(zero_ints, dim3((ng + 255) / 256), dim3(256), 0, cs,
                                (int *)(g->dev + st.off_tickets), ng);
-            err = launch_groups(plan, st, g->dev, cs);
+            err = launch_groups(plan, st, g->dev, cs, &side);
         }
         hipGraph_t graph = nullptr;
         hipError_t ce = hipStreamEndCapture(cs, &graph);
@@ -1498,6 +1595,7 @@ void *BQCgraph_capture(int nmol, BasisProdCache **bps, double **vj, double **vk,
     if (!err && hipGraphInstantiate(&g->exec, g->graph, nullptr, nullptr, 0) != hipSuccess) err = 1;
     g_prof = was_prof;
     if (cs) hipStreamDestroy(cs);
+    side.destroy();
     if (err) {
         if (g->graph) hipGraphDestroy(g->graph);
         if (g->dev) hipFree(g->dev);
