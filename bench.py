@@ -125,9 +125,11 @@ KIND_NAMES = {0: 'jk_quartets', 1: 'jk_rows', 4: 'jk_wave'}
 def kernel_name(cls, kind, split=False):
     """Template name of a profiled launch: class code li*1000+lj*100+lk*10+ll,
     kind 0 quartet / 1 row / 4 wavefront kernel, +2 for the FP32 instance, +8
-    for the b-side pass of a split row class.  split names the a-side and
+    for the b-side pass of a split row class, +16 for the tile row kernel.  split names the a-side and
     b-side row kernels of a class together."""
     ls = (cls // 1000, cls // 100 % 10, cls // 10 % 10, cls % 10)
+    if kind & 16:
+        return 'jk_tile<%d,%d,%d,%d>' % ls
     t = 'float' if kind & 2 else 'double'
     if split:
         return ' + '.join('%s<%d,%d,%d,%d,%s,%d>' % (KIND_NAMES[1], *ls, t, r) for r in (1, 2))
@@ -508,7 +510,7 @@ def main():
     ap.add_argument('--no-cpu', action='store_true')
     ap.add_argument('--row-split', type=int, default=-1, choices=(-1, 0, 1),
                     help='two-pass (a-side / b-side) digestion of the small s/p row classes: '
-                         '-1 the built-in per-class rule, 0 none, 1 every candidate')
+                         '-1 the built-in rule (none), 0 none, 1 every candidate')
     ap.add_argument('--persistent', type=int, default=2, choices=(0, 1, 2),
                     help='persistent work-queue grids for the row kernels: '
                          '0 never, 1 for molecules from 2048 Cartesian AOs, 2 always (default)')

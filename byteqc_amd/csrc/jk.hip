@@ -60,7 +60,8 @@ static thread_local double g_last_flops[2] = {0, 0};
 // on the build's stream.  Records (class code, algorithmic FLOPs, events).
 struct LaunchRec {
     int cls;       // li*1000 + lj*100 + lk*10 + ll of the evaluated class
-    int kind;      // 0 quartet kernel, 1 row kernel, 4 wave kernel; +2 for FP32
+    int kind;      // 0 quartet kernel, 1 row kernel, 4 wave kernel; +2 for FP32,
+                   // +8 for the b-side pass, +16 for the tile kernel (17)
     double flops;  // algorithmic FLOPs of the launch
     double nquart;
     hipEvent_t e0, e1;
@@ -460,17 +461,20 @@ static int tile_for(int kind, int cls, int prec, int nao, bool *fixed = nullptr)
 }
 
 // Orders of the pair lists of a plan by first shell (which = 0; for the
-// reference-ABI entry GINTbuild_jk, whose caller has no such array) and by
-// second shell (which = 1; the b-side lists of split row classes): per pair
-// type the plan positions sorted by that shell, stable (a counting sort of a
-// row of the host bas_pair2shls, which the cache aliases).  Built per pair
+// reference-ABI entry GINTbuild_jk, whose caller has no such array), by
+// second shell (which = 1; the b-side lists of split row classes) and by
+// blocks of BQC_PAIR_BLOCK first and second shells, inside a block by first
+// shell (which = 2; the Q lists of the tile kernels): per pair type the plan
+// positions in that order, stable (sorts of rows of the host bas_pair2shls,
+// which the cache aliases).  Built per pair
 // type on first use and kept per cache until BQCdel_basis_prod_clone or
 // GINTdel_basis_prod forgets it.
+#define BQC_PAIR_BLOCK 16
 struct PairOrder {
     const int *pair2shls = nullptr;
     int npairs = 0, ncptype = 0;
-    std::vector<int> order[2];
-    std::vector<char> done[2];
+    std::vector<int> order[3];
+    std::vector<char> done[3];
 };
 static std::mutex g_order_mu;
 static std::map<const BasisProdCache *, PairOrder> g_orders;
@@ -485,7 +489,7 @@ static const int *shell_order(const BasisProdCache *bp, int which, int cp_a, int
         po.pair2shls = bp->bas_pair2shls;
         po.npairs = npairs;
         po.ncptype = bp->ncptype;
-        for (int w = 0; w < 2; ++w) {
+        for (int w = 0; w < 3; ++w) {
             po.order[w].assign(npairs > 0 ? npairs : 1, 0);
             po.done[w].assign(bp->ncptype, 0);
         }
@@ -494,6 +498,20 @@ static const int *shell_order(const BasisProdCache *bp, int which, int cp_a, int
     for (int cp : cps) {
         if (po.done[which][cp]) continue;
         const int p0 = locs[cp], n = locs[cp + 1] - locs[cp];
+        if (which == 2) {
+            const int *k1 = bp->bas_pair2shls + p0, *k2 = k1 + npairs;
+            std::vector<std::pair<unsigned long long, int>> v(n);
+            for (int k = 0; k < n; ++k)
+                v[k] = {(unsigned long long)(k1[k] / BQC_PAIR_BLOCK) << 48 |
+                            (unsigned long long)(k2[k] / BQC_PAIR_BLOCK) << 32 |
+                            (unsigned long long)(k1[k] % BQC_PAIR_BLOCK) << 16 |
+                            (unsigned long long)(k2[k] % BQC_PAIR_BLOCK),
+                        k};
+            std::sort(v.begin(), v.end());
+            for (int k = 0; k < n; ++k) po.order[2][p0 + k] = v[k].second;
+            po.done[2][cp] = 1;
+            continue;
+        }
         const int *key = bp->bas_pair2shls + (which ? npairs : 0) + p0;
         int lo = 0, hi = -1;
         for (int k = 0; k < n; ++k) {
@@ -514,20 +532,18 @@ extern "C" void bqc_forget_pair_order(const BasisProdCache *bp) {
     g_orders.erase(bp);
 }
 
-// Split row classes (a-side and b-side passes) by class code; -1 entries are
-// unset (default on).  Set by BQCset_row_split.
+// Split row classes (a-side and b-side passes) by class code.  Set by
+// BQCset_row_split.
 #define BQC_SPLIT_MAX 64
 static int g_split_cls[BQC_SPLIT_MAX], g_split_val[BQC_SPLIT_MAX], g_split_n = 0;
-static int g_split_all = -1;  // -1: the built-in per-class rule
+static int g_split_all = -1;  // -1: the built-in rule
 static bool split_on(int cls) {
     for (int i = 0; i < g_split_n; ++i)
         if (g_split_cls[i] == cls) return g_split_val[i] != 0;
-    if (g_split_all >= 0) return g_split_all != 0;
-    // measured per class on MI355X (64 waters cc-pVDZ, 128 waters cc-pVTZ):
-    // (ps|ps) ran 20 ms faster in one pass on the larger molecule and equal
-    // on the smaller, (dp|ss) 0.5 ms faster on the smaller; the other split
-    // candidates gain 1-150 ms from the two passes
-    return cls != 1010 && cls != 2100;
+    // off unless asked for: jk_tile is faster than the two passes of every
+    // candidate but (pp|ss) and (dp|ss) on 64 waters cc-pVDZ (6.6 and 3.6
+    // against 6.6 and 3.8 ms), where it ties
+    return g_split_all > 0;
 }
 
 template <class T> using StdVec = std::vector<T>;
@@ -580,14 +596,24 @@ static void side_order(const int *bins, int nbins, const int *order, int npairs_
     }
 }
 
-// Kernels of a task per precision: the row kernel of the class when there is
-// one within the scratch and LDS limits, else the wave kernel.  False if a
+static bool is_tile(RowKernel k) {
+    for (int a = 0; a < BQC_NPAIRID; ++a)
+        for (int b = 0; b <= a; ++b)
+            if (k && g_rows[3][0][a][b] == k) return true;
+    return false;
+}
+
+// Kernels of a task per precision: the tile or row kernel of the class when
+// there is one within the scratch and LDS limits, else the wave kernel.  False if a
 // precision has neither (the generic kernels take the task).  *log_cut: the
 // precision rule with a row class that has no FP32 instance kept in FP64.
 static bool pick_kernels(const TaskCtx &c, RowKernel (&k)[2], int (&wv)[2], double *log_cut) {
     *log_cut = c.log_cut;
     for (int prec = 0; prec < 2; ++prec) {
-        RowKernel r = c.swap ? g_rows[0][prec][c.pkl][c.pij] : g_rows[0][prec][c.pij][c.pkl];
+        auto row = [&](int role) {
+            return c.swap ? g_rows[role][prec][c.pkl][c.pij] : g_rows[role][prec][c.pij][c.pkl];
+        };
+        RowKernel r = row(3) ? row(3) : row(0);
         RowKernel w = c.swap ? g_waves[prec][c.pkl][c.pij] : g_waves[prec][c.pij][c.pkl];
         if (r && scratch_ok((const void *)r)) {
             k[prec] = r;
@@ -747,6 +773,16 @@ static int plan_task(BuildPlanT<V> &bp_, const TaskCtx &c, const int *bra_order,
     td.nprim_q = bp->cptype[cp_q].nprim_12;
     td.diag = c.diag;
     td.nbins = nbins;
+    // Q list of a tile kernel by blocks of shells across the bins (the kernel
+    // takes the pairs below each P bin's limit): 64 Q pairs then share 35
+    // shells instead of 56.  For the classes whose time goes to flushing the
+    // block, in items long enough to fill it: 64 waters cc-pVDZ (ss|ss) 11.3
+    // -> 9.6 ms, (ps|ss) 17.2 -> 14.4, 12 molecules def2-SVP (ps|ss) 27.0 ->
+    // 25.5; (ps|ps) loses 0.6 ms there and gains 0.7 here, (pp|ps) loses 0.8,
+    // and short items only gather more (8 waters 2.6 -> 2.9 ms).
+    const bool blocks = is_tile(k[0]) && class_components(eval_cls(c)) <= 9 && !t_noalloc &&
+                        log_cut <= -1e299 && bp->bas_pair2shls &&
+                        item_tile(load, c, k[0], 0, 0, jk.nao) >= 32;
     bp_.tasks.push_back(td);
     bp_.bins_off.push_back(bp_.ints.size());
     bp_.ints.insert(bp_.ints.end(), pbins, pbins + nbins + 1);
@@ -754,7 +790,12 @@ static int plan_task(BuildPlanT<V> &bp_, const TaskCtx &c, const int *bra_order,
     size_t off_p = bp_.ints.size();
     side_order(pbins, nbins, bra_order + locs[cp_p], locs[cp_p + 1] - locs[cp_p], bp_.ints);
     size_t off_q = off_p;
-    if (cp_p != cp_q) {
+    if (blocks) {
+        off_q = bp_.ints.size();
+        const int *order = shell_order(bp, 2, cp_q, cp_q) + locs[cp_q];
+        for (int q = 0; q < locs[cp_q + 1] - locs[cp_q]; ++q)
+            if (order[q] < nq) bp_.ints.push_back(order[q]);
+    } else if (cp_p != cp_q) {
         off_q = bp_.ints.size();
         side_order(qbins, nbins, bra_order + locs[cp_q], locs[cp_q + 1] - locs[cp_q], bp_.ints);
     }
@@ -793,11 +834,15 @@ static int plan_task(BuildPlanT<V> &bp_, const TaskCtx &c, const int *bra_order,
                 int rmax;
                 q_limits(p & ~63, rmax, qsplit);
             }
+            if (blocks && (prec || qmax == 0)) continue;
+            // list positions of the item: all of a block list, of which the
+            // fraction qmax / nq is taken
             const int lo = prec ? qsplit : 0;
-            const int hi = prec ? qmax : (qsplit < qmax ? qsplit : qmax);
+            const int hi = blocks ? nq : (prec ? qmax : (qsplit < qmax ? qsplit : qmax));
+            const int len = blocks ? (int)std::min<long long>(nq, ((long long)ck * nq + qmax - 1) / qmax) : ck;
             const int pitem = wv[prec] ? p : p / 64;
-            for (int q0 = lo; q0 < hi; q0 += ck) {
-                int q1 = q0 + ck < hi ? q0 + ck : hi;
+            for (int q0 = lo; q0 < hi; q0 += len) {
+                int q1 = q0 + len < hi ? q0 + len : hi;
                 it.push_back(ti);
                 it.push_back(pitem);
                 it.push_back(q0);
@@ -837,6 +882,8 @@ static int plan_task(BuildPlanT<V> &bp_, const TaskCtx &c, const int *bra_order,
     return 0;
 }
 
+#define BQC_TICKET_INTS (BQC_TICKET_SLICES * BQC_TICKET_STRIDE)
+
 // Device image of a BuildPlan: [TaskDesc array][list orders][items].
 template <template <class> class V>
 struct StagedT {
@@ -853,8 +900,8 @@ static StagedT<V> stage_layout(const BuildPlanT<V> &p) {
     size_t off = align16(p.tasks.size() * sizeof(TaskDesc));
     st.off_perm = off;
     off = align16(off + p.ints.size() * sizeof(int));
-    st.off_tickets = off;  // work counters, BQC_TICKET_SLICES per group, zero in the image
-    off = align16(off + p.groups.size() * BQC_TICKET_SLICES * sizeof(int));
+    st.off_tickets = off;  // work counters, BQC_TICKET_INTS per group, zero in the image
+    off = align16(off + p.groups.size() * BQC_TICKET_INTS * sizeof(int));
     st.off_qrec = off;     // Q list records, written on the device
     off = align16(off + p.nqrec * sizeof(int4));
     for (const GroupT<V> &g : p.groups) {
@@ -878,7 +925,7 @@ static void stage_fill(BuildPlanT<V> &p, const StagedT<V> &st, char *dev, char *
     }
     memcpy(host, p.tasks.data(), p.tasks.size() * sizeof(TaskDesc));
     memcpy(host + st.off_perm, p.ints.data(), p.ints.size() * sizeof(int));
-    memset(host + st.off_tickets, 0, p.groups.size() * BQC_TICKET_SLICES * sizeof(int));
+    memset(host + st.off_tickets, 0, p.groups.size() * BQC_TICKET_INTS * sizeof(int));
     for (size_t gi = 0; gi < p.groups.size(); ++gi)
         memcpy(host + st.off_items[gi], p.groups[gi].items.data(),
                p.groups[gi].items.size() * sizeof(int));
@@ -917,13 +964,13 @@ static int launch_group(const BuildPlanT<V> &p, const StagedT<V> &st, char *dev,
         const unsigned cap = resident_blocks((const void *)g.kern, (int)nthr);
         if (cap > 0 && cap < nblk) {
             nblk = cap;
-            ticket = (int *)(dev + st.off_tickets) + gi * BQC_TICKET_SLICES;
+            ticket = (int *)(dev + st.off_tickets) + gi * BQC_TICKET_INTS;
         }
     }
     LaunchRec rec;
     if (prof_on())
-        record_launch(rec, g.cls, (g.wave ? 4 : 1) + 2 * g.prec + 8 * g.role_b, g.flops, g.nquart,
-                      stream);
+        record_launch(rec, g.cls, (g.wave ? 4 : 1) + 2 * g.prec + 8 * g.role_b + (is_tile(g.kern) ? 16 : 0),
+                      g.flops, g.nquart, stream);
     hipLaunchKernelGGL(g.kern, dim3(nblk), dim3(nthr), 0, stream, (const TaskDesc *)dev, items,
                        nitems, ticket);
     if (prof_on()) keep_launch(rec, stream);
@@ -1582,7 +1629,7 @@ void *BQCgraph_capture(int nmol, BasisProdCache **bps, double **vj, double **vk,
         plan.flops[1] += fl[1];
         if (!err && !plan.groups.empty()) {
             // replays start from zero work counters (a kernel, not a memset)
-            const int ng = (int)plan.groups.size() * BQC_TICKET_SLICES;
+            const int ng = (int)plan.groups.size() * BQC_TICKET_INTS;
             hipLaunchKernelGGL(zero_ints, dim3((ng + 255) / 256), dim3(256), 0, cs,
                                (int *)(g->dev + st.off_tickets), ng);
             err = launch_groups(plan, st, g->dev, cs, &side);

@@ -113,7 +113,13 @@ __device__ __forceinline__ void atomic_add(gdouble *p, double v) {
 // XN consecutive Cartesian components of shell a starting at x0 are
 // evaluated (XN = NFI: the whole block); gout holds XN*NFJ*NFK*NFL values.
 // rys_tab: nullptr (table in global memory) or a pointer to the table of
-// this class's root count in LDS.
+// this class's root count in LDS (rys_stage).
+// A primitive quartet of (ps|ss) is some 95 FP64 instructions in dependent
+// chains, and the wavefronts that fit beside the accumulators do not hide the
+// latencies: so the Q data of the next one are loaded ahead, divisions and
+// square roots are 4-6 instructions, and the Rys polynomials run as parallel
+// chains (12 molecules def2-SVP, all classes: 215 -> 202 ms from the short
+// reciprocals, 187 -> 181 from the loads ahead and the parallel chains).
 template <int LA, int LB, int LC, int LD, typename T, int XN = Cls<LA, LB, LC, LD>::NFI,
           typename RysPtr = std::nullptr_t>
 __device__ __forceinline__ void eri_block(T *__restrict__ gout, const PairData &pd,
@@ -144,23 +150,31 @@ __device__ __forceinline__ void eri_block(T *__restrict__ gout, const PairData &
         const double eij = pre ? p_first[1] : pe12[p];
         const double P[3] = {pre ? p_first[2] : px12[p], pre ? p_first[3] : py12[p],
                              pre ? p_first[4] : pz12[p]};
+        // the next Q primitive pair is loaded while this one is used
+        double nakl = qa12[qq0], nekl = qe12[qq0], nQ[3] = {qx12[qq0], qy12[qq0], qz12[qq0]};
         for (int iq = 0; iq < np_q; ++iq) {
-            const int q = qq0 + iq;
-            const double akl = qa12[q], ekl = qe12[q];
-            const double Q[3] = {qx12[q], qy12[q], qz12[q]};
+            const double akl = nakl, ekl = nekl;
+            const double Q[3] = {nQ[0], nQ[1], nQ[2]};
+            const int qn = qq0 + (iq + 1 < np_q ? iq + 1 : iq);
+            nakl = qa12[qn];
+            nekl = qe12[qn];
+            nQ[0] = qx12[qn];
+            nQ[1] = qy12[qn];
+            nQ[2] = qz12[qn];
             const double pq[3] = {P[0] - Q[0], P[1] - Q[1], P[2] - Q[2]};
             const double aijkl = aij + akl;
             const double a1 = aij * akl;
-            const double a0 = a1 / aijkl;
+            const double rs = fast_rsqrt(aijkl);
+            const double a0 = a1 * (rs * rs);
             const double x = a0 * (pq[0] * pq[0] + pq[1] * pq[1] + pq[2] * pq[2]);
             double u[NR], w[NR];
             if constexpr (std::is_same<RysPtr, std::nullptr_t>::value) rys_roots<NR>(x, u, w);
             else rys_roots<NR>(x, u, w, rys_tab);
-            const double fac = eij * ekl / (sqrt(aijkl) * a1);
+            const double fac = eij * ekl * rs * fast_rcp(a1);
 #pragma unroll
             for (int r = 0; r < NR; ++r) {
                 const double u2 = a0 * u[r];
-                const double tmp4 = 0.5 / (u2 * aijkl + a1);
+                const double tmp4 = 0.5 * fast_rcp(fma(u2, aijkl, a1));
                 const double b00 = u2 * tmp4;
                 const double b10 = b00 + tmp4 * akl;
                 const double b01 = b00 + tmp4 * aij;
@@ -203,7 +217,7 @@ __device__ __forceinline__ void eri_block(T *__restrict__ gout, const PairData &
             // Not in the classes above 81 components, whose registers are
             // full: there the test added spills ((dp|ds) 240 -> 268 ms).
             if constexpr (C::NF <= 81)
-                if (iq + 1 < np_q && qe12[q + 1] == 0.0) break;
+                if (nekl == 0.0) break;
         }
         if constexpr (C::NF <= 81)
             if (ip + 1 < np_p && pe12[p + 1] == 0.0) break;

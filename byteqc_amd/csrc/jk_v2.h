@@ -30,11 +30,14 @@
 #pragma once
 #include "jk_kernel.h"
 
-#define BQC_V2_CK 64
+// Most roots whose table the row kernels stage in LDS
+#define BQC_RYS_LDS_MAX 4
 // Work counters per persistent launch: the item list is cut into this many
 // contiguous slices, one per XCD (workgroups are dispatched to the XCDs in
 // turn, so workgroup b runs on XCD b % 8)
 #define BQC_TICKET_SLICES 8
+// ints between two counters: each in a 128-byte line of its own
+#define BQC_TICKET_STRIDE 32
 
 // Cross-lane moves of a double through DPP (two 32-bit halves).  Lanes
 // whose source is outside the pattern, or whose row is masked off, read 0.
@@ -134,10 +137,50 @@ constexpr int row_pack_max() {
                 max2(pack_nv(NA * NC), pack_nv(NB * NC)));
 }
 
-// Work item: (task, chunk of 64 P pairs, first and end Q position).  With
-// ticket == NULL wavefront w of block b takes item 4b + w; otherwise the grid
-// is persistent and the wavefronts pull items from the counter *ticket
-// (zero before the launch).
+// Work items of one wavefront of a launch of 256-lane workgroups.  Without
+// counters (ticket == NULL) wavefront w of block b takes item 4b + w; else the
+// grid is persistent and the wavefronts take items until the list is
+// exhausted.  A wavefront starts on the list slice of its XCD, so the items an
+// XCD runs together are neighbours in the list (nearby shells: their density
+// reads and J/K atomics share that XCD's L2).  Once the slice is exhausted it
+// reads all counters (zero before the launch) with one load and moves to the
+// next slice that has items left: trying the others in turn queues up 8
+// atomics per wavefront at the end of every launch, 0.2 ms with 3072
+// wavefronts when the counters share a line.
+struct ItemQueue {
+    int *ticket;
+    int nitems, slice;
+    bool first = true;
+    __device__ ItemQueue(int *t, int n) : ticket(t), nitems(n), slice(blockIdx.x % BQC_TICKET_SLICES) {}
+    __device__ int lo(int s) const { return (int)((long long)nitems * s / BQC_TICKET_SLICES); }
+    // the next item, or nitems if none is left
+    __device__ int next() {
+        if (!ticket) {
+            const int it = first ? (int)(blockIdx.x * 4 + (threadIdx.x >> 6)) : nitems;
+            first = false;
+            return __builtin_amdgcn_readfirstlane(it);
+        }
+        const int lane = threadIdx.x & 63;
+        for (;;) {
+            int got = 0;
+            if (lane == 0)
+                got = __hip_atomic_fetch_add(ticket + slice * BQC_TICKET_STRIDE, 1,
+                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const int it = lo(slice) + __builtin_amdgcn_readfirstlane(got);
+            if (it < lo(slice + 1)) return it;
+            const int s = lane & (BQC_TICKET_SLICES - 1);
+            const int taken = __hip_atomic_load(ticket + s * BQC_TICKET_STRIDE, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT);
+            unsigned left = (unsigned)__ballot(lo(s) + taken < lo(s + 1)) & 0xffu;
+            if (!left) return nitems;
+            // the first slice with items left after the current one
+            left |= left << 8;
+            slice = (slice + __builtin_ctz(left >> slice)) % BQC_TICKET_SLICES;
+        }
+    }
+};
+
+// Work item: (task, chunk of 64 P pairs, first and end Q position).
 template <int LA, int LB, int LC, int LD, typename T, int ROLE = 0>
 __global__ void __launch_bounds__(256)
     jk_rows(const TaskDesc *__restrict__ tasks, const int4 *__restrict__ items, int nitems,
@@ -145,17 +188,15 @@ __global__ void __launch_bounds__(256)
     using C = Cls<LA, LB, LC, LD>;
     constexpr int NA = C::NFI, NB = C::NFJ, NC = C::NFK, ND = C::NFL;
     // Rys interpolation table of this class's root count staged in LDS
-    // (8 KB for 1 root, 20 KB for 2) before any wave leaves
-    constexpr bool RYS_LDS = C::NR <= 2;
-    constexpr int RYS_N = RYS_LDS ? rys_table_size(C::NR) : 1;
-    __shared__ double rys_lds[RYS_N];
-    if (RYS_LDS) {
-        const double *src = BQC_RYS_COEF + rys_offset(C::NR);
-        for (int i = threadIdx.x; i < RYS_N; i += blockDim.x) rys_lds[i] = src[i];
+    // (9, 21, 36, 53 KB for 1 to 4 roots) before any wave leaves
+    constexpr bool RYS_LDS = C::NR <= BQC_RYS_LDS_MAX;
+    constexpr int RYS_N = RYS_LDS ? rys_lds_size(C::NR) : 2;
+    __shared__ __align__(16) double rys_lds[RYS_N];
+    if constexpr (RYS_LDS) {
+        rys_stage<C::NR, 256>(rys_lds);
         __syncthreads();
     }
-    typedef const __attribute__((address_space(3))) double *lds_ptr;
-    const lds_ptr rys_tab = (lds_ptr)rys_lds;
+    const rys_lds_ptr rys_tab = (rys_lds_ptr)rys_lds;
     // per-wavefront staging of packed atomics
     constexpr int PK = row_pack_max<NA, NB, NC, ND>();
     __shared__ double pk_val[4 * 64 * (PK > 0 ? PK : 1)];
@@ -470,39 +511,16 @@ __global__ void __launch_bounds__(256)
             }
         }
     };
-    // one work item per wavefront, or (persistent grids) items taken from
-    // the slice counters until the list is exhausted: a wavefront starts on
-    // the slice of its XCD, so the items an XCD runs together are neighbours
-    // in the list (nearby shells: their density reads and J/K atomics share
-    // that XCD's L2), and moves on to the next slice when its own is empty.
-    // One call site keeps the item's code inlined once.
-    int slice = blockIdx.x % BQC_TICKET_SLICES, tries = 0;
-    auto next_item = [&]() -> int {
-        if (!ticket) return __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
-        while (tries < BQC_TICKET_SLICES) {
-            const int lo = (int)((long long)nitems * slice / BQC_TICKET_SLICES);
-            const int hi = (int)((long long)nitems * (slice + 1) / BQC_TICKET_SLICES);
-            int tk0 = 0;
-            if ((threadIdx.x & 63) == 0)
-                tk0 = __hip_atomic_fetch_add(ticket + slice, 1, __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT);
-            const int it = lo + __builtin_amdgcn_readfirstlane(tk0);
-            if (it < hi) return it;
-            slice = slice + 1 == BQC_TICKET_SLICES ? 0 : slice + 1;
-            ++tries;
-        }
-        return nitems;
-    };
-    for (int item = next_item(); item < nitems; item = next_item()) {
-        run_item(item);
-        if (!ticket) break;
-    }
+    // one call site keeps the item's code inlined once
+    ItemQueue queue(ticket, nitems);
+    for (int item = queue.next(); item < nitems; item = queue.next()) run_item(item);
 }
 
 typedef void (*RowKernel)(const TaskDesc *, const int4 *, int, int *);
 // [role][precision][bra pair id][ket pair id]: role 0 the single pass, roles
-// 1 and 2 the a-side and b-side passes of split classes (FP64 only)
-typedef RowKernel RowKernelTable[3][2][BQC_NPAIRID][BQC_NPAIRID];
+// 1 and 2 the a-side and b-side passes of split classes (FP64 only), 3 the
+// tile kernel (FP64 only, jk_tile.h)
+typedef RowKernel RowKernelTable[4][2][BQC_NPAIRID][BQC_NPAIRID];
 
 // Classes digested with the wavefront-stationary kernel, per precision.
 // Up to 108 Cartesian components the FP64 block and the lane accumulators
@@ -534,17 +552,4 @@ constexpr bool row_fp32() {
 template <int LA, int LB, int LC, int LD>
 constexpr bool row_split_candidate() {
     return Cls<LA, LB, LC, LD>::NF <= 27 && LA <= 2 && LC <= 1;
-}
-
-template <int LA, int LB, int LC, int LD>
-static void reg_row(RowKernelTable &tab) {
-    constexpr int pab = LA * (LA + 1) / 2 + LB, pcd = LC * (LC + 1) / 2 + LD;
-    if constexpr (use_rows<LA, LB, LC, LD, double>())
-        tab[0][0][pab][pcd] = jk_rows<LA, LB, LC, LD, double>;
-    if constexpr (use_rows<LA, LB, LC, LD, float>() && row_fp32<LA, LB, LC, LD>())
-        tab[0][1][pab][pcd] = jk_rows<LA, LB, LC, LD, float>;
-    if constexpr (use_rows<LA, LB, LC, LD, double>() && row_split_candidate<LA, LB, LC, LD>()) {
-        tab[1][0][pab][pcd] = jk_rows<LA, LB, LC, LD, double, 1>;
-        tab[2][0][pab][pcd] = jk_rows<LA, LB, LC, LD, double, 2>;
-    }
 }

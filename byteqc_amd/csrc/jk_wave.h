@@ -20,7 +20,7 @@
 // workgroup barriers.
 #pragma once
 #include "digest_split.h"
-#include "jk_v2.h"
+#include "jk_tile.h"
 
 template <int LA, int LB, int LC, int LD>
 struct WaveCls {
@@ -254,7 +254,8 @@ __global__ void __launch_bounds__(64, (wave_min_waves<LA, LB, LC, LD>()))
                         const double akl = ua12[qq], ekl = ue12[qq];
                         const double Q[3] = {ux12[qq], uy12[qq], uz12[qq]};
                         const double pq[3] = {P[0] - Q[0], P[1] - Q[1], P[2] - Q[2]};
-                        const double aijkl = aij + akl, a1 = aij * akl, a0q = a1 / aijkl;
+                        const double aijkl = aij + akl, a1 = aij * akl;
+                        const double rs = fast_rsqrt(aijkl), a0q = a1 * (rs * rs);
                         const double x = a0q * (pq[0] * pq[0] + pq[1] * pq[1] + pq[2] * pq[2]);
                         // phase A: one (direction, root) table per lane
                         if (lane < 3 * NR) {
@@ -262,12 +263,12 @@ __global__ void __launch_bounds__(64, (wave_min_waves<LA, LB, LC, LD>()))
                             double ur, wr;
                             rys_root_one<NR>(x, r, ur, wr);
                             const double u2 = a0q * ur;
-                            const double tmp4 = 0.5 / (u2 * aijkl + a1);
+                            const double tmp4 = 0.5 * fast_rcp(fma(u2, aijkl, a1));
                             const double b00 = u2 * tmp4;
                             const double b10 = b00 + tmp4 * akl;
                             const double b01 = b00 + tmp4 * aij;
                             const double seed = d == 0 ? norm
-                                                : (d == 1 ? eij * ekl / (sqrt(aijkl) * a1) : wr);
+                                                : (d == 1 ? eij * ekl * rs * fast_rcp(a1) : wr);
                             const double Pd = d == 0 ? P[0] : (d == 1 ? P[1] : P[2]);
                             const double Qd = d == 0 ? Q[0] : (d == 1 ? Q[1] : Q[2]);
                             const double Ad = d == 0 ? ra[0] : (d == 1 ? ra[1] : ra[2]);

@@ -207,9 +207,8 @@ int BQCset_tile(int kind, int cls, int prec, int ck);
  * builds use them for molecules from 2048 Cartesian AOs up (below that the
  * doubled integral work cost more than the atomics saved: 256 molecules of
  * 4-40 waters took 7.2 s against 5.5 s per batch).  on: 0 or 1; for
- * cls = -1 also -1, the built-in rule (the default): two passes for every
- * candidate but (ps|ps) and (dp|ss), which measured as fast or faster in one
- * pass on MI355X.  Process-wide; not to be called while another thread plans
+ * cls = -1 also -1, the built-in rule (the default): one pass of the tile
+ * kernel for every class, which measured as fast or faster on MI355X.  Process-wide; not to be called while another thread plans
  * a build.  No counterpart in the reference.  Returns 0 ok, 1 bad argument or
  * too many per-class settings. */
 int BQCset_row_split(int cls, int on);
@@ -292,7 +291,8 @@ int BQCsymmetrize_jk(double *vj, double *vk, int nao, int n_dm, hipStream_t stre
  * kernel launch is bracketed by HIP events on the build's stream.
  * BQCprofile_read drains the records (waiting for their events): per launch
  * the evaluated class li*1000+lj*100+lk*10+ll, the kernel kind (0 quartet
- * kernel, 1 row kernel), the algorithmic FLOPs and quartet count of the
+ * kernel, 1 row kernel, 4 wavefront kernel; + 2 FP32, + 8 b-side pass, + 16
+ * tile kernel), the algorithmic FLOPs and quartet count of the
  * launch and its duration in ms; returns the number written (<= cap). */
 void BQCprofile_enable(int on);
 int BQCprofile_count(void);
