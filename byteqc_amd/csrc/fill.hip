@@ -69,6 +69,7 @@ extern "C" int GINTfill_int2e(BasisProdCache *bp, double *eri, int nao, const in
     pd.bra = bp->bas_pair2bra;
     pd.ket = bp->bas_pair2ket;
     pd.ao_loc = bp->ao_loc;
+    pd.prec = nullptr;
     TaskArgs ta;
     const int cp_p = swap ? cp_kl_id : cp_ij_id, cp_q = swap ? cp_ij_id : cp_kl_id;
     auto reset = [&]() {

@@ -392,8 +392,17 @@ static int launch_quartets(const TaskCtx &c, const JKArgs &jk, const PairData &p
     return 0;
 }
 
+// Device records of the primitive pairs of a cache (BQCset_prim_records).
+static std::mutex g_prec_mu;
+static std::map<const BasisProdCache *, const double *> g_precs;
+
 static PairData make_pair_data(const BasisProdCache *bp) {
     PairData pd;
+    {
+        std::lock_guard<std::mutex> lock(g_prec_mu);
+        const auto it = g_precs.find(bp);
+        pd.prec = it == g_precs.end() ? nullptr : it->second;
+    }
     pd.a12 = bp->a12;
     pd.e12 = bp->e12;
     pd.x12 = bp->x12;
@@ -528,6 +537,10 @@ static const int *shell_order(const BasisProdCache *bp, int which, int cp_a, int
 }
 
 extern "C" void bqc_forget_pair_order(const BasisProdCache *bp) {
+    {
+        std::lock_guard<std::mutex> lock(g_prec_mu);
+        g_precs.erase(bp);
+    }
     std::lock_guard<std::mutex> lock(g_order_mu);
     g_orders.erase(bp);
 }
@@ -1714,6 +1727,14 @@ int BQCset_row_split(int cls, int on) {
     if (g_split_n >= BQC_SPLIT_MAX) return 1;
     g_split_cls[g_split_n] = cls;
     g_split_val[g_split_n++] = on;
+    return 0;
+}
+
+int BQCset_prim_records(BasisProdCache *bpcache, const double *records) {
+    if (!bpcache) return 1;
+    std::lock_guard<std::mutex> lock(g_prec_mu);
+    if (records) g_precs[bpcache] = records;
+    else g_precs.erase(bpcache);
     return 0;
 }
 

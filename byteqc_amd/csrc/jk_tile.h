@@ -135,9 +135,14 @@ __global__ void __launch_bounds__(256, (TileCls<LA, LB, LC, LD>::WAVES))
             b0 = lao[sb];
             ra[0] = lbx[sa]; ra[1] = lby[sa]; ra[2] = lbz[sa];
             rb[0] = lbx[sb]; rb[1] = lby[sb]; rb[2] = lbz[sb];
-            p_first[0] = glb(pd.a12)[pp0]; p_first[1] = glb(pd.e12)[pp0];
-            p_first[2] = glb(pd.x12)[pp0]; p_first[3] = glb(pd.y12)[pp0];
-            p_first[4] = glb(pd.z12)[pp0];
+            if (pd.prec) {
+#pragma unroll
+                for (int k = 0; k < 5; ++k) p_first[k] = glb(pd.prec)[(size_t)pp0 * BQC_PREC + k];
+            } else {
+                p_first[0] = glb(pd.a12)[pp0]; p_first[1] = glb(pd.e12)[pp0];
+                p_first[2] = glb(pd.x12)[pp0]; p_first[3] = glb(pd.y12)[pp0];
+                p_first[4] = glb(pd.z12)[pp0];
+            }
         }
         // rows of the block: NA per distinct a, then NB per distinct b.  If
         // they leave no room for the columns of one Q pair, the lanes take

@@ -364,6 +364,14 @@ class _VHFOpt:
                                     _ptr(d['bas_coords']), _ptr(d['aexyz']),
                                     _ptr(d['pair2shls']))
         self.bpcache = bpg
+        if (self.cp_nprim > 1).any():
+            # one record per primitive pair for the kernels' per-lane reads;
+            # finished here, because builds may run on other streams
+            rec = torch.zeros((nprim_pairs, 8), dtype=torch.float64, device=dev)
+            rec[:, :5] = d['aexyz'].view(5, -1).T
+            torch.cuda.current_stream().synchronize()
+            d['prim_records'] = rec
+            lib.BQCset_prim_records(bpg, _ptr(rec))
         self.coeff_dev = torch.as_tensor(self.coeff, device=dev)
 
     def clear(self):

@@ -213,6 +213,15 @@ int BQCset_tile(int kind, int cls, int prec, int ck);
  * too many per-class settings. */
 int BQCset_row_split(int cls, int on);
 
+/* Device records of a cache's primitive pairs: 8 doubles per pair, in the
+ * order of aexyz, the first five a12, e12, x12, y12, z12 (64-byte aligned).
+ * The lanes of the row kernels read the pairs of different shell pairs, one
+ * after the other: one line of a record instead of five lines of the arrays.
+ * bpcache: the device clone; records must stay valid while builds use the
+ * clone and may be NULL (the arrays are read).  Forgotten with the clone.  No
+ * counterpart in the reference.  Returns 0 ok, 1 bad argument. */
+int BQCset_prim_records(BasisProdCache *bpcache, const double *records);
+
 /* Launch shape of the row kernels.  Persistent grids have as many
  * workgroups as fit on the device at once, each wavefront pulling work items
  * from a counter in the build's work list until it is exhausted; the other
