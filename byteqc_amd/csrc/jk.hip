@@ -1020,6 +1020,27 @@ struct SideStreams {
         }
         return dev == d;
     }
+    // The side streams' work from here on runs after what the stream holds
+    int begin(hipStream_t stream) {
+        if (hipEventRecord(fork, stream) != hipSuccess) return 1;
+        for (int i = 0; i < BQC_SIDE_STREAMS; ++i)
+            if (hipStreamWaitEvent(s[i], fork, 0) != hipSuccess) return 1;
+        return 0;
+    }
+    // and the stream's work from here on after theirs.
+    int end(hipStream_t stream) {
+        int err = 0;
+        for (int i = 0; i < BQC_SIDE_STREAMS; ++i)
+            if (hipEventRecord(join[i], s[i]) != hipSuccess ||
+                hipStreamWaitEvent(stream, join[i], 0) != hipSuccess)
+                err = 1;
+        return err;
+    }
+    // Index of the stream with the least queued: 0 the build's own, i the
+    // side stream i - 1.
+    static int least(const double *queued) {
+        return (int)(std::min_element(queued, queued + BQC_SIDE_STREAMS + 1) - queued);
+    }
     void destroy() {
         for (int i = 0; i < BQC_SIDE_STREAMS; ++i) {
             if (s[i]) (void)hipStreamDestroy(s[i]);
@@ -1058,20 +1079,14 @@ static int launch_groups(const BuildPlanT<V> &p, const StagedT<V> &st, char *dev
                      gi};
     std::sort(order.begin(), order.end());
     double queued[BQC_SIDE_STREAMS + 1] = {};
-    if (hipEventRecord(side->fork, stream) != hipSuccess) return 1;
-    for (int i = 0; i < BQC_SIDE_STREAMS; ++i)
-        if (hipStreamWaitEvent(side->s[i], side->fork, 0) != hipSuccess) return 1;
+    if (side->begin(stream)) return 1;
     int err = 0;
     for (const auto &o : order) {
-        const int k = (int)(std::min_element(queued, queued + BQC_SIDE_STREAMS + 1) - queued);
+        const int k = side->least(queued);
         queued[k] -= o.first;
         err |= launch_group(p, st, dev, o.second, k ? side->s[k - 1] : stream);
     }
-    for (int i = 0; i < BQC_SIDE_STREAMS; ++i)
-        if (hipEventRecord(side->join[i], side->s[i]) != hipSuccess ||
-            hipStreamWaitEvent(stream, side->join[i], 0) != hipSuccess)
-            err = 1;
-    return err;
+    return side->end(stream) ? 1 : err;
 }
 
 // Device images of the work lists of direct (non-graph) builds: a ring of
@@ -1296,18 +1311,19 @@ static int check_build_args(const MolArgs *m, int nmol, int nbins, int precision
 }
 
 // Direct builds: tasks grouped by integral class (classes in order of first
-// appearance, tasks in order inside a class).  Below BQC_SPREAD_FLOPS all
-// classes are planned into one work list (one copy, one fill_qrec) and their
-// launches spread over several streams: a launch ends with some 0.1-0.3 ms of
-// a few long items, and launches of small molecules are nothing but that, so
-// the next class fills the chip meanwhile (ms on MI355X, one stream -> four: 4
-// waters def2-SVP 7.1 -> 5.1, 8 waters cc-pVDZ 4.0 -> 2.9, 5 waters cc-pVTZ
-// 16.1 -> 9.3, 24 waters cc-pVTZ 177 -> 165, 12 molecules def2-SVP 255 -> 250,
-// 64 waters cc-pVDZ 120 -> 120).  Above, each class is staged and launched as
-// soon as it is planned, so the device runs the first classes while the host
-// plans the rest (128 waters cc-pVTZ, 4e13 FLOPs: a launch's end is below 1 %
-// of it, planning ahead of all launches would not be hidden).
-#define BQC_SPREAD_FLOPS 4e12
+// appearance, tasks in order inside a class), their launches on the stream and
+// its side streams: a launch ends with some 0.1-0.3 ms of a few long items,
+// and launches of small molecules are nothing but that, so the next class
+// fills the chip meanwhile (ms on MI355X, one stream -> four: 4 waters def2-SVP
+// 7.1 -> 5.1, 8 waters cc-pVDZ 4.0 -> 2.9, 5 waters cc-pVTZ 16.1 -> 9.3, 24
+// waters cc-pVTZ 177 -> 165).  Below BQC_ONE_LIST_FLOPS all classes are
+// planned into one work list (one copy, one fill_qrec: 1 water cc-pVDZ 1.05 ->
+// 0.85 ms, 5 waters cc-pVTZ 7.7 -> 7.2).  Above, each class is staged and
+// launched as soon as it is planned, so the device runs the first classes
+// while the host plans the rest (one list -> class by class: 12 molecules
+// def2-SVP 211 -> 186, 64 waters cc-pVDZ 93.9 -> 88.6, 40 waters def2-SVP
+// mixed 52.3 -> 48.9).
+#define BQC_ONE_LIST_FLOPS 1e11
 static int build_by_class(const MolArgs *m, int nmol, int nbins, int precision, double fp32_cut,
                           hipStream_t stream, double flops[2]) {
     flops[0] = flops[1] = 0;
@@ -1332,24 +1348,34 @@ static int build_by_class(const MolArgs *m, int nmol, int nbins, int precision, 
             }
             by_cls[k].push_back(TaskRef{im, t});
         }
-    const bool spread = work < BQC_SPREAD_FLOPS;
-    if (spread && by_cls.size() > 1) {
+    const bool one_list = work < BQC_ONE_LIST_FLOPS;
+    if (one_list && by_cls.size() > 1) {
         for (size_t k = 1; k < by_cls.size(); ++k)
             by_cls[0].insert(by_cls[0].end(), by_cls[k].begin(), by_cls[k].end());
         by_cls.resize(1);
     }
-    for (const std::vector<TaskRef> &list : by_cls) {
+    // classes in turn on the stream and its side streams, each to the one
+    // with the least work queued so far
+    SideStreams &side = stage_for(stream).side;
+    const bool rotate = !one_list && by_cls.size() > 1 && !prof_on() && side.ready();
+    double queued[BQC_SIDE_STREAMS + 1] = {};
+    if (rotate && side.begin(stream)) return 1;
+    err = 0;
+    for (size_t k = 0; k < by_cls.size() && !err; ++k) {
         BuildPlan plan;
         std::vector<Deferred> def;
-        err = plan_list(plan, m, list.data(), list.size(), nbins, precision, fp32_cut, def);
+        err = plan_list(plan, m, by_cls[k].data(), by_cls[k].size(), nbins, precision, fp32_cut,
+                        def);
         for (Deferred &d : def)
             if (!err) err = launch_quartets(d.c, d.jk, d.pd, stream, plan.flops);
-        if (!err) err = stage_and_launch(plan, stream, spread);
+        const int on = rotate ? side.least(queued) : 0;
+        queued[on] += plan.flops[0] + plan.flops[1];
+        if (!err) err = stage_and_launch(plan, on ? side.s[on - 1] : stream, one_list);
         flops[0] += plan.flops[0];
         flops[1] += plan.flops[1];
-        if (err) return err;
     }
-    return 0;
+    if (rotate && side.end(stream) && !err) err = 1;
+    return err;
 }
 
 // Plans all tasks of all molecules.  Classes without row/wave kernels go to
