@@ -421,18 +421,22 @@ def dm_cond_batch(dmcs, locs, stream=None):
     """Block bounds max|D| over (group, group) AO blocks for device matrices
     dmcs[m] (nao_m x nao_m) with group AO offsets locs[m]; returns host arrays."""
     dev = dmcs[0].device
+    n = len(dmcs)
     ng = numpy.array([len(l) - 1 for l in locs], dtype=numpy.int32)
     off = numpy.append(0, numpy.cumsum([len(l) for l in locs]))[:-1].astype(numpy.int32)
     outoff = numpy.append(0, numpy.cumsum(ng * ng))[:-1].astype(numpy.int32)
-    ptrs = torch.tensor([m.data_ptr() for m in dmcs], dtype=torch.int64, device=dev)
-    nao = torch.tensor([m.shape[-1] for m in dmcs], dtype=torch.int32, device=dev)
-    loc_d = torch.as_tensor(numpy.concatenate(locs).astype(numpy.int32), device=dev)
-    off_d = torch.as_tensor(off, device=dev)
-    ng_d = torch.as_tensor(ng, device=dev)
-    oo_d = torch.as_tensor(outoff, device=dev)
+    # pointers, sizes and offsets in one copy: [ptrs | nao | off | ng | outoff | loc]
+    ints = numpy.concatenate([[m.shape[-1] for m in dmcs], off, ng, outoff, *locs]).astype(
+        numpy.int32)
+    arg = numpy.zeros(8 * n + 4 * len(ints), dtype=numpy.uint8)
+    arg[:8 * n].view(numpy.int64)[:] = [m.data_ptr() for m in dmcs]
+    arg[8 * n:].view(numpy.int32)[:] = ints
+    arg_d = torch.as_tensor(arg, device=dev)
+    base = arg_d.data_ptr()
+    ptrs = ctypes.c_void_p(base)
+    nao, off_d, ng_d, oo_d, loc_d = (ctypes.c_void_p(base + 8 * n + 4 * n * k) for k in range(5))
     out = torch.zeros(int((ng * ng).sum()), dtype=torch.float64, device=dev)
-    err = load_library().BQCdm_cond(_ptr(ptrs), _ptr(nao), _ptr(loc_d), _ptr(off_d), _ptr(ng_d),
-                                    _ptr(oo_d), _ptr(out), len(dmcs), int(ng.max()),
+    err = load_library().BQCdm_cond(ptrs, nao, loc_d, off_d, ng_d, oo_d, _ptr(out), n, int(ng.max()),
                                     max(int(m.shape[-1]) for m in dmcs), _stream_ptr(stream))
     if err:
         raise RuntimeError('density bound kernel failed')
