@@ -686,6 +686,7 @@ static void add_load(ClassLoad &load, const TaskCtx &c) {
         steps[0] += (wv[0] ? np : np / 64.0) * qsplit;
         steps[1] += (wv[1] ? np : np / 64.0) * (qmax - qsplit);
     }
+    if (is_tile(k[0])) steps[0] *= tile_parts(eval_cls(c));
     for (int prec = 0; prec < 2; ++prec) load.at(c, prec) += steps[prec] * step_cost(c);
 }
 
@@ -707,19 +708,36 @@ static void add_load(ClassLoad &load, const TaskCtx &c) {
 #define BQC_FILL_HI 8
 #define BQC_FILL_LO 0.25
 #define BQC_ITEM_MIN 96
+// share: work of the launch relative to what load holds.
 static int item_tile(ClassLoad &load, const TaskCtx &c, RowKernel kern, int wave, int prec,
-                     int nao) {
+                     int nao, double share = 1) {
     bool fixed;
     const int cap = tile_for(wave ? 4 : 1, eval_cls(c), prec, nao, &fixed);
     if (fixed) return cap;
     const unsigned waves = wave ? resident_blocks((const void *)kern, 64)
                                 : 4 * resident_blocks((const void *)kern, 256);
     if (!waves) return cap;
-    const double per_wave = load.at(c, prec) / waves;
+    const double per_wave = share * load.at(c, prec) / waves;
     const double cost = std::max(per_wave / BQC_FILL_HI,
                                  std::min(per_wave / BQC_FILL_LO, (double)BQC_ITEM_MIN));
     const double ck = cost / step_cost(c);
     return ck >= cap ? cap : (ck > 1 ? (int)ck : 1);
+}
+
+// The wavefront kernel of a class whose tile kernel takes five or six parts, if
+// the launch is too small for those: 64 quartets a step, each evaluated once
+// per part, leave the device empty where one quartet per wavefront does not.
+// The line is 50 uncontracted steps per resident wavefront: 64 waters cc-pVDZ
+// (dd|pp) with 46 took 1.46 ms in parts against 1.14, (dd|ds) with 38 1.32
+// against 0.70, (dp|dp) with 60 1.40 against 1.98.
+#define BQC_PARTS_MIN_LOAD (50 * (1 + BQC_STEP_BASE))
+static RowKernel small_parts_kernel(const TaskCtx &c, RowKernel tile, ClassLoad &load) {
+    if (!is_tile(tile) || tile_parts(eval_cls(c)) <= 2) return nullptr;
+    RowKernel w = c.swap ? g_waves[0][c.pkl][c.pij] : g_waves[0][c.pij][c.pkl];
+    const unsigned waves = 4 * resident_blocks((const void *)tile, 256);
+    if (!w || !scratch_ok((const void *)w) || load.at(c, 0) >= (double)BQC_PARTS_MIN_LOAD * waves)
+        return nullptr;
+    return w;
 }
 
 // Adds one task to the plan; load holds the work of the whole launch set.
@@ -732,6 +750,12 @@ static int plan_task(BuildPlanT<V> &bp_, const TaskCtx &c, const int *bra_order,
     int wv[2];
     double log_cut;
     if (!pick_kernels(c, k, wv, &log_cut)) return -1;
+    double share = 1;
+    if (RowKernel w = small_parts_kernel(c, k[0], load)) {
+        k[0] = w;
+        wv[0] = 1;
+        share = 64.0 / tile_parts(eval_cls(c));
+    }
     // split row class: a-side and b-side passes (FP64 builds of the class only)
     RowKernel ks[2] = {nullptr, nullptr};
     const int *order2 = nullptr;
@@ -836,8 +860,9 @@ static int plan_task(BuildPlanT<V> &bp_, const TaskCtx &c, const int *bra_order,
     // pair holds for every pair of the row in both precisions, so the two
     // precisions cover each pair's Q range exactly once.
     const bool by_row = !wv[0] || !wv[1];
+    const int parts = is_tile(k[0]) ? tile_parts(cls) : 1;
     for (int prec = 0; prec < 2; ++prec) {
-        const int ck = item_tile(load, c, k[prec], wv[prec], prec, jk.nao);
+        const int ck = item_tile(load, c, k[prec], wv[prec], prec, jk.nao, prec ? 1 : share);
         const int step = wv[prec] ? 1 : 64;
         V<int> &it = g[prec]->items;
         for (int p = 0; p < np; p += step) {
@@ -856,10 +881,12 @@ static int plan_task(BuildPlanT<V> &bp_, const TaskCtx &c, const int *bra_order,
             const int pitem = wv[prec] ? p : p / 64;
             for (int q0 = lo; q0 < hi; q0 += len) {
                 int q1 = q0 + len < hi ? q0 + len : hi;
-                it.push_back(ti);
-                it.push_back(pitem);
-                it.push_back(q0);
-                it.push_back(q1);
+                for (int part = 0; part < (prec ? 1 : parts); ++part) {
+                    it.push_back(ti);
+                    it.push_back(pitem | part << BQC_PART_SHIFT);
+                    it.push_back(q0);
+                    it.push_back(q1);
+                }
             }
         }
     }

@@ -39,6 +39,9 @@ using namespace bqc;
 #define BQC_THREADS 256
 // Largest Cartesian AO count: J/K/D element offsets are 32-bit in the kernels
 #define BQC_MAX_NAO 46340
+// Part of a tile-kernel item (see tile_parts), in the high bits of its chunk
+#define BQC_PART_SHIFT 28
+#define BQC_PART_MASK ((1 << BQC_PART_SHIFT) - 1)
 
 struct TaskArgs {
     int bas_p0, bas_q0;    // first global pair index of the p / q side
@@ -128,8 +131,10 @@ __device__ __forceinline__ void atomic_add(gdouble *p, double v) {
 // reciprocals, 187 -> 181 from the loads ahead and the parallel chains).  The
 // P pairs of a wavefront's lanes lie apart: their records take 64 lines of L1
 // per primitive instead of 320 (181 -> 175 ms, 40 waters mixed 52.5 -> 50.1).
+// FLAT: all loops unrolled (needs a compile-time x0), so that the block stays
+// in registers.
 template <int LA, int LB, int LC, int LD, typename T, int XN = Cls<LA, LB, LC, LD>::NFI,
-          typename RysPtr = std::nullptr_t>
+          typename RysPtr = std::nullptr_t, bool FLAT = !Cls<LA, LB, LC, LD>::BIG>
 __device__ __forceinline__ void eri_block(T *__restrict__ gout, const PairData &pd,
                                           int pp0, int np_p, int qq0, int np_q, double norm,
                                           const double *ra, const double *rb,
@@ -139,7 +144,8 @@ __device__ __forceinline__ void eri_block(T *__restrict__ gout, const PairData &
     using C = Cls<LA, LB, LC, LD>;
     constexpr int NR = C::NR;
     constexpr int NG = XN * C::NFJ * C::NFK * C::NFL;
-#pragma unroll C::UN
+    constexpr int UO = FLAT ? 16 : 1, UN = FLAT ? 2048 : 8;
+#pragma unroll UN
     for (int n = 0; n < NG; ++n) gout[n] = (T)0;
     const double ab[3] = {ra[0] - rb[0], ra[1] - rb[1], ra[2] - rb[2]};
     const double cd[3] = {rc[0] - rd[0], rc[1] - rd[1], rc[2] - rd[2]};
@@ -215,11 +221,11 @@ __device__ __forceinline__ void eri_block(T *__restrict__ gout, const PairData &
                 rys2d<LA, LB, LC, LD, T>(Iz, (T)w[r], (T)((P[2] - ra[2]) - tmp2 * pq[2]),
                                          (T)((Q[2] - rc[2]) + tmp3 * pq[2]), (T)b10, (T)b01,
                                          (T)b00, (T)ab[2], (T)cd[2]);
-#pragma unroll C::UO
+#pragma unroll UO
                 for (int x = 0; x < XN; ++x) {
                     const int ax = cart_x(LA, x0 + x), ay = cart_y(LA, x0 + x),
                               az = cart_z(LA, x0 + x);
-#pragma unroll C::UO
+#pragma unroll UO
                     for (int y = 0; y < C::NFJ; ++y) {
                         const int bx = cart_x(LB, y), by = cart_y(LB, y), bz = cart_z(LB, y);
 #pragma unroll
@@ -239,12 +245,12 @@ __device__ __forceinline__ void eri_block(T *__restrict__ gout, const PairData &
             // the pair builder sorts primitive pairs by |e12| and zeroes the
             // negligible ones: stop before the next one if it is zero (tested
             // after the work, so single-primitive pairs never wait on it).
-            // Not in the classes above 81 components, whose registers are
+            // Not in blocks above 81 components, whose registers are
             // full: there the test added spills ((dp|ds) 240 -> 268 ms).
-            if constexpr (C::NF <= 81)
+            if constexpr (NG <= 81)
                 if (nekl == 0.0) break;
         }
-        if constexpr (C::NF <= 81)
+        if constexpr (NG <= 81)
             if (ip + 1 < np_p &&
                 (pd.prec ? glb(pd.prec)[(size_t)(p + 1) * BQC_PREC + 1] : pe12[p + 1]) == 0.0)
                 break;

@@ -1,4 +1,5 @@
-// Row kernel with its exchange block in LDS: the FP64 row classes.
+// Row kernel with its exchange block in LDS: the FP64 kernel of the classes up
+// to 324 components (in parts above 54).
 //
 // As in jk_rows a wavefront owns 64 pairs (a b) of the P list and walks a
 // range of the Q list in lock-step, and the six digestion sums are the same.
@@ -25,15 +26,46 @@
 #pragma once
 #include "jk_v2.h"
 
+// Parts that the Cartesian components of shell a of class code c are dealt
+// into, each part an item of its own (0: no tile kernel).  The blocks of the
+// larger classes do not fit the 512 registers of a lane; a part's does, at the
+// price of its recurrences being evaluated once per part.  All digestion sums
+// are linear in the components of a, so a part is a shell with fewer
+// components.  Measured on MI355X (24 waters cc-pVTZ, ms, one block or the
+// wavefront kernel -> parts): two parts (dp|pp) 9.9 -> 2.9 (12 molecules
+// def2-SVP 21.3 -> 6.3), (dp|ds) 5.8 -> 2.7, (dd|ps) 4.8 -> 1.9, (fp|ps) 2.9 ->
+// 1.7, (ff|ss) 2.4 -> 0.8, (fs|fs) 2.3 -> 0.4, (fs|pp) 1.5 -> 1.0, (fd|ss) 1.4
+// -> 0.9, (fs|ds) 1.4 -> 1.0; five (fs|dp) 4.1 -> 2.1, (fp|ds) 4.1 -> 1.8,
+// (fd|ps) 3.7 -> 1.9, (fp|pp) 3.5 -> 1.9, (fp|fs) 1.8 -> 1.0; six (dp|dp) 7.5 ->
+// 4.0, (dd|ds) 3.9 -> 2.4, (dd|pp) 3.3 -> 2.4.  Not so (dd|dp) 4.0 -> 8.0,
+// (fd|ds) 2.3 -> 3.5, (fd|pp) 2.1 -> 2.3, and hardly (fp|dp) 4.4 -> 3.6,
+// (fs|dd) 1.4 -> 1.2, (ff|ps) 1.4 -> 1.1 (5 waters 0.20 -> 0.28, 0.11 -> 0.24).
+constexpr int tile_parts(int c) {
+    switch (c) {
+        case 2111: case 2120: case 2210: case 3011: case 3110: case 3300: case 3030: case 3020:
+        case 3200:
+            return 2;
+        case 3021: case 3120: case 3210: case 3111: case 3130:
+            return 5;
+        case 2121: case 2211: case 2220:
+            return 6;
+    }
+    return ncart(c / 1000) * ncart(c / 100 % 10) * ncart(c / 10 % 10) * ncart(c % 10) <= 81 ? 1 : 0;
+}
+template <int LA, int LB, int LC, int LD>
+constexpr int tile_parts() { return tile_parts(LA * 1000 + LB * 100 + LC * 10 + LD); }
+
 template <int LA, int LB, int LC, int LD>
 struct TileCls {
     using C = Cls<LA, LB, LC, LD>;
-    static constexpr int NA = C::NFI, NB = C::NFJ, NC = C::NFK, ND = C::NFL;
+    static constexpr int PARTS = tile_parts<LA, LB, LC, LD>() > 0 ? tile_parts<LA, LB, LC, LD>() : 1;
+    static constexpr int NA = C::NFI / PARTS, NB = C::NFJ, NC = C::NFK, ND = C::NFL;
+    static constexpr int NF = NA * NB * NC * ND;
     // resident wavefronts per SIMD, and so workgroups per CU: what registers
     // allow with few spills.  (pp|ps) runs 20.3 ms with one and no spills, 15.8
     // with two and 95 spilled registers (12 molecules def2-SVP); (ps|ss) 27.6
     // with two, 24.2 with three.
-    static constexpr int WAVES = C::NF <= 3 ? 3 : (C::NF <= 27 ? 2 : 1);
+    static constexpr int WAVES = NF <= 3 ? 3 : (NF <= 27 ? 2 : 1);
     // doubles of LDS per wavefront for the block of K: what WAVES workgroups
     // per CU leave of 160 KB after the Rys table and the row and column lists
     static constexpr int CAP = (163840 / WAVES - rys_lds_size(C::NR) * 8 -
@@ -69,6 +101,15 @@ __device__ __forceinline__ unsigned long long distinct_firsts(int key, unsigned 
     return firsts;
 }
 
+// f(0), f(1), ... f(N - 1) with compile-time arguments.
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void each_part(F f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>());
+        each_part<N, I + 1>(f);
+    }
+}
+
 __device__ __forceinline__ void lds_add(double *p, double v) {
     __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
@@ -93,11 +134,11 @@ __global__ void __launch_bounds__(256, (TileCls<LA, LB, LC, LD>::WAVES))
     // records of the gathered Q pairs, in the block's memory before it is set
     int *const recs = (int *)tile;
 
-    auto run_item = [&](const int item) {
-        const int4 it = items[item];
+    auto run_item = [&](const int4 it, auto part_c) {
+        constexpr int X0 = decltype(part_c)::value * NA;  // first component of a
         const TaskDesc &tk = tasks[__builtin_amdgcn_readfirstlane(it.x)];
         const PairData &pd = tk.pd;
-        const int chunk = __builtin_amdgcn_readfirstlane(it.y);
+        const int chunk = __builtin_amdgcn_readfirstlane(it.y & BQC_PART_MASK);
         const int q0 = __builtin_amdgcn_readfirstlane(it.z);
         const int qe = __builtin_amdgcn_readfirstlane(it.w);
         // neighbours in the list (which share a) sit 16 lanes apart: one LDS
@@ -131,7 +172,7 @@ __global__ void __launch_bounds__(256, (TileCls<LA, LB, LC, LD>::WAVES))
         double ra[3] = {0, 0, 0}, rb[3] = {0, 0, 0};
         double p_first[5] = {1, 0, 0, 0, 0};
         if (pvalid) {
-            a0 = lao[sa];
+            a0 = lao[sa] + X0;
             b0 = lao[sb];
             ra[0] = lbx[sa]; ra[1] = lby[sa]; ra[2] = lbz[sa];
             rb[0] = lbx[sb]; rb[1] = lby[sb]; rb[2] = lbz[sb];
@@ -312,18 +353,18 @@ __global__ void __launch_bounds__(256, (TileCls<LA, LB, LC, LD>::WAVES))
                             }
                         }
                     }
-                    double g[C::NF];
+                    double g[TC::NF];
                     if (active) {
                         const int qq0 =
                             __builtin_amdgcn_readfirstlane(tk.prim_q0 + qpos * tk.nprim_q);
                         const double rc[3] = {ubx[sc], uby[sc], ubz[sc]};
                         const double rd[3] = {ubx[sd], uby[sd], ubz[sd]};
-                        eri_block<LA, LB, LC, LD, double>(g, pd, pp0, tk.nprim_p, qq0,
-                                                          tk.nprim_q, norm, ra, rb, rc, rd, 0,
-                                                          rys_tab, p_first);
+                        eri_block<LA, LB, LC, LD, double, NA, rys_lds_ptr, true>(
+                            g, pd, pp0, tk.nprim_p, qq0, tk.nprim_q, norm, ra, rb, rc, rd, X0,
+                            rys_tab, p_first);
                     } else {
 #pragma unroll
-                        for (int k = 0; k < C::NF; ++k) g[k] = 0.0;
+                        for (int k = 0; k < TC::NF; ++k) g[k] = 0.0;
                     }
 #define G(x, y, z, w) g[(((x) * NB + (y)) * NC + (z)) * ND + (w)]
                     if (do_j) {
@@ -423,25 +464,29 @@ __global__ void __launch_bounds__(256, (TileCls<LA, LB, LC, LD>::WAVES))
         }
     };
     ItemQueue queue(ticket, nitems);
-    for (int item = queue.next(); item < nitems; item = queue.next()) run_item(item);
+    for (int item = queue.next(); item < nitems; item = queue.next()) {
+        const int4 it = items[item];
+        const int part = __builtin_amdgcn_readfirstlane((unsigned)it.y >> BQC_PART_SHIFT);
+        each_part<TC::PARTS>([&](auto c) {
+            if (part == decltype(c)::value) run_item(it, c);
+        });
+    }
 }
 
-// Row classes with a tile instance: all but (dp|ds), whose 919 spilled
-// registers make it slower than jk_rows (7.6 against 5.8 ms on 24 waters
-// cc-pVTZ), and (fs|fs), whose block does not fit.
+// Classes with a tile instance.
 template <int LA, int LB, int LC, int LD>
 constexpr bool use_tile() {
-    if constexpr (use_rows<LA, LB, LC, LD, double>())
-        return TileCls<LA, LB, LC, LD>::FITS && LA * 1000 + LB * 100 + LC * 10 + LD != 2120;
+    if constexpr (tile_parts<LA, LB, LC, LD>() > 0) return TileCls<LA, LB, LC, LD>::FITS;
     return false;
 }
 
 template <int LA, int LB, int LC, int LD>
 static void reg_row(RowKernelTable &tab) {
     constexpr int pab = LA * (LA + 1) / 2 + LB, pcd = LC * (LC + 1) / 2 + LD;
-    if constexpr (use_tile<LA, LB, LC, LD>())
+    if constexpr (use_tile<LA, LB, LC, LD>()) {
+        static_assert(ncart(LA) % tile_parts<LA, LB, LC, LD>() == 0, "parts of equal size");
         tab[3][0][pab][pcd] = jk_tile<LA, LB, LC, LD>;
-    else if constexpr (use_rows<LA, LB, LC, LD, double>())
+    } else if constexpr (use_rows<LA, LB, LC, LD, double>())
         tab[0][0][pab][pcd] = jk_rows<LA, LB, LC, LD, double>;
     if constexpr (use_rows<LA, LB, LC, LD, float>() && row_fp32<LA, LB, LC, LD>())
         tab[0][1][pab][pcd] = jk_rows<LA, LB, LC, LD, float>;
