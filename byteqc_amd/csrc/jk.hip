@@ -705,6 +705,7 @@ static void add_load(ClassLoad &load, const TaskCtx &c) {
 // 0.5: 32.8 / 27.0 / 26.7 for 5 waters cc-pVTZ, 4.6 / 4.1 / 4.8 for 8 waters
 // cc-pVDZ; BQC_ITEM_MIN 24 / 48 / 96 / 192: 12.6 / 11.8 / 11.8 / 13.8 for 13
 // waters cc-pVDZ with two densities.
+#define BQC_TILE_ITEM 256
 #define BQC_FILL_HI 8
 #define BQC_FILL_LO 0.25
 #define BQC_ITEM_MIN 96
@@ -712,8 +713,12 @@ static void add_load(ClassLoad &load, const TaskCtx &c) {
 static int item_tile(ClassLoad &load, const TaskCtx &c, RowKernel kern, int wave, int prec,
                      int nao, double share = 1) {
     bool fixed;
-    const int cap = tile_for(wave ? 4 : 1, eval_cls(c), prec, nao, &fixed);
+    int cap = tile_for(wave ? 4 : 1, eval_cls(c), prec, nao, &fixed);
     if (fixed) return cap;
+    // the tile kernels' set-up is longer than the row kernels' whose bands
+    // these are: 32 / 64 / 128 / 256 / 512 took 89.0 / 79.8 / 76.9 / 76.1 / 76.7
+    // ms on 64 waters cc-pVDZ, within 1 % elsewhere
+    if (is_tile(kern)) cap = BQC_TILE_ITEM;
     const unsigned waves = wave ? resident_blocks((const void *)kern, 64)
                                 : 4 * resident_blocks((const void *)kern, 256);
     if (!waves) return cap;
