@@ -125,14 +125,14 @@ KIND_NAMES = {0: 'jk_quartets', 1: 'jk_rows', 4: 'jk_wave'}
 def kernel_name(cls, kind, split=False):
     """Template name of a profiled launch: class code li*1000+lj*100+lk*10+ll,
     kind 0 quartet / 1 row / 4 wavefront kernel, +2 for the FP32 instance, +8
-    for the b-side pass of a split row class, +16 for the tile row kernel.  split names the a-side and
-    b-side row kernels of a class together."""
+    for the b-side pass of a split row class, +16 for the tile kernel.  split
+    names the a-side and b-side row kernels of a class together."""
     ls = (cls // 1000, cls // 100 % 10, cls // 10 % 10, cls % 10)
     if kind & 16:
         return 'jk_tile<%d,%d,%d,%d>' % ls
     t = 'float' if kind & 2 else 'double'
     if split:
-        return ' + '.join('%s<%d,%d,%d,%d,%s,%d>' % (KIND_NAMES[1], *ls, t, r) for r in (1, 2))
+        return ' + '.join('jk_rows<%d,%d,%d,%d,%d>' % (*ls, r) for r in (1, 2))
     return '%s<%d,%d,%d,%d,%s>' % (KIND_NAMES[kind & ~10], *ls, t)
 
 
@@ -146,10 +146,7 @@ def measured_traffic(workload, kernel):
     with open(path) as f:
         rec = json.load(f)
     kernels = rec.get('kernels', {})
-    # the profiler names a one-pass row kernel with its role argument (0)
     k = kernels.get(kernel)
-    if k is None and kernel.startswith('jk_rows<') and kernel.count(',') == 4:
-        k = kernels.get(kernel[:-1] + ',0>')
     return None if k is None else float(k['hbm_bytes_per_launch'])
 
 

@@ -612,35 +612,30 @@ static void side_order(const int *bins, int nbins, const int *order, int npairs_
 static bool is_tile(RowKernel k) {
     for (int a = 0; a < BQC_NPAIRID; ++a)
         for (int b = 0; b <= a; ++b)
-            if (k && g_rows[3][0][a][b] == k) return true;
+            if (k && g_rows[0][a][b] == k) return true;
     return false;
 }
 
-// Kernels of a task per precision: the tile or row kernel of the class when
-// there is one within the scratch and LDS limits, else the wave kernel.  False if a
-// precision has neither (the generic kernels take the task).  *log_cut: the
-// precision rule with a row class that has no FP32 instance kept in FP64.
+// Kernels of a task per precision: the tile kernel of the class when there is
+// one within the scratch and LDS limits, else the wave kernels.  False if
+// there is neither (the generic kernels take the task).  *log_cut: the
+// precision rule, with every quartet in FP64 where the class has a tile kernel
+// or no FP32 instance (FP64 code for k[1] then, with no items).
 static bool pick_kernels(const TaskCtx &c, RowKernel (&k)[2], int (&wv)[2], double *log_cut) {
+    auto usable = [&](const auto &t) {
+        const RowKernel r = c.swap ? t[c.pkl][c.pij] : t[c.pij][c.pkl];
+        return r && scratch_ok((const void *)r) ? r : nullptr;
+    };
     *log_cut = c.log_cut;
-    for (int prec = 0; prec < 2; ++prec) {
-        auto row = [&](int role) {
-            return c.swap ? g_rows[role][prec][c.pkl][c.pij] : g_rows[role][prec][c.pij][c.pkl];
-        };
-        RowKernel r = row(3) ? row(3) : row(0);
-        RowKernel w = c.swap ? g_waves[prec][c.pkl][c.pij] : g_waves[prec][c.pij][c.pkl];
-        if (r && scratch_ok((const void *)r)) {
-            k[prec] = r;
-            wv[prec] = 0;
-        } else if (w && scratch_ok((const void *)w)) {
-            k[prec] = w;
-            wv[prec] = 1;
-        } else if (prec == 1 && !wv[0]) {
-            k[1] = k[0];
-            wv[1] = 0;
-            *log_cut = -1e300;
-        } else {
-            return false;
-        }
+    k[0] = usable(g_rows[0]);
+    wv[0] = !k[0];
+    if (!k[0]) k[0] = usable(g_waves[0]);
+    if (!k[0]) return false;
+    k[1] = wv[0] ? usable(g_waves[1]) : nullptr;
+    wv[1] = wv[0];
+    if (!k[1]) {
+        k[1] = k[0];
+        *log_cut = -1e300;
     }
     return true;
 }
@@ -757,8 +752,8 @@ static int plan_task(BuildPlanT<V> &bp_, const TaskCtx &c, const int *bra_order,
     if (!pick_kernels(c, k, wv, &log_cut)) return -1;
     double share = 1;
     if (RowKernel w = small_parts_kernel(c, k[0], load)) {
-        k[0] = w;
-        wv[0] = 1;
+        k[0] = k[1] = w;
+        wv[0] = wv[1] = 1;
         share = 64.0 / tile_parts(eval_cls(c));
     }
     // split row class: a-side and b-side passes (FP64 builds of the class only)
@@ -767,7 +762,7 @@ static int plan_task(BuildPlanT<V> &bp_, const TaskCtx &c, const int *bra_order,
     if (!wv[0] && !t_noalloc && log_cut <= -1e299 && jk.nao >= BQC_TILE_BIG_NAO &&
         split_on(eval_cls(c)) && c.bp->bas_pair2shls) {
         for (int role = 1; role <= 2; ++role)
-            ks[role - 1] = c.swap ? g_rows[role][0][c.pkl][c.pij] : g_rows[role][0][c.pij][c.pkl];
+            ks[role - 1] = c.swap ? g_rows[role][c.pkl][c.pij] : g_rows[role][c.pij][c.pkl];
         if (ks[0] && ks[1] && scratch_ok((const void *)ks[0]) && scratch_ok((const void *)ks[1])) {
             const int cp_p = c.swap ? c.cp_kl : c.cp_ij;
             order2 = shell_order(c.bp, 1, cp_p, cp_p);
@@ -861,10 +856,6 @@ static int plan_task(BuildPlanT<V> &bp_, const TaskCtx &c, const int *bra_order,
         qmax = qbins[nbins - s];
         qsplit = qbins[fp32_split(c, cp_p, cp_q, pbins, qbins, s, log_cut)];
     };
-    // When one precision runs rows of 64 P pairs, the split of a row's first
-    // pair holds for every pair of the row in both precisions, so the two
-    // precisions cover each pair's Q range exactly once.
-    const bool by_row = !wv[0] || !wv[1];
     const int parts = is_tile(k[0]) ? tile_parts(cls) : 1;
     for (int prec = 0; prec < 2; ++prec) {
         const int ck = item_tile(load, c, k[prec], wv[prec], prec, jk.nao, prec ? 1 : share);
@@ -873,10 +864,6 @@ static int plan_task(BuildPlanT<V> &bp_, const TaskCtx &c, const int *bra_order,
         for (int p = 0; p < np; p += step) {
             int qmax, qsplit;
             q_limits(p, qmax, qsplit);
-            if (by_row && (p & 63)) {
-                int rmax;
-                q_limits(p & ~63, rmax, qsplit);
-            }
             if (blocks && (prec || qmax == 0)) continue;
             // list positions of the item: all of a block list, of which the
             // fraction qmax / nq is taken

@@ -483,15 +483,14 @@ constexpr bool use_tile() {
 template <int LA, int LB, int LC, int LD>
 static void reg_row(RowKernelTable &tab) {
     constexpr int pab = LA * (LA + 1) / 2 + LB, pcd = LC * (LC + 1) / 2 + LD;
+    static_assert(use_tile<LA, LB, LC, LD>() || Cls<LA, LB, LC, LD>::NF > 81,
+                  "the wave kernels start above 81 components");
     if constexpr (use_tile<LA, LB, LC, LD>()) {
         static_assert(ncart(LA) % tile_parts<LA, LB, LC, LD>() == 0, "parts of equal size");
-        tab[3][0][pab][pcd] = jk_tile<LA, LB, LC, LD>;
-    } else if constexpr (use_rows<LA, LB, LC, LD, double>())
-        tab[0][0][pab][pcd] = jk_rows<LA, LB, LC, LD, double>;
-    if constexpr (use_rows<LA, LB, LC, LD, float>() && row_fp32<LA, LB, LC, LD>())
-        tab[0][1][pab][pcd] = jk_rows<LA, LB, LC, LD, float>;
-    if constexpr (use_rows<LA, LB, LC, LD, double>() && row_split_candidate<LA, LB, LC, LD>()) {
-        tab[1][0][pab][pcd] = jk_rows<LA, LB, LC, LD, double, 1>;
-        tab[2][0][pab][pcd] = jk_rows<LA, LB, LC, LD, double, 2>;
+        tab[0][pab][pcd] = jk_tile<LA, LB, LC, LD>;
+    }
+    if constexpr (row_split_candidate<LA, LB, LC, LD>()) {
+        tab[1][pab][pcd] = jk_rows<LA, LB, LC, LD, 1>;
+        tab[2][pab][pcd] = jk_rows<LA, LB, LC, LD, 2>;
     }
 }

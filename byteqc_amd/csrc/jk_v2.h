@@ -15,23 +15,20 @@
 //   K(a,c) += g D(b,d)    lane register accumulator over a run of equal c,
 //                         flushed by a segmented sum over runs of equal a
 //   K(a,d) += g D(b,c)    segmented sum over runs of equal a at every step
-//   K(b,c) += g D(a,d)    lane register accumulator over a run of equal c
-//   K(b,d) += g D(a,c)    one atomic per lane and component (smallest block)
+//   K(b,c) += g D(a,d)    as K(a,c), K(a,d) for runs of equal b
+//   K(b,d) += g D(a,c)
 //
 // The per-lane K(b,c), K(b,d) atomics dominate the atomic requests of the
-// small s/p classes.  For those classes every quartet can instead be
-// evaluated twice: by the a-side instance (ROLE 1: J(a,b), J(c,d), K(a,c),
-// K(a,d)) over P lists sorted by a, and by the b-side instance (ROLE 2:
-// K(b,c), K(b,d), as register sums over runs of equal c flushed by segmented
-// sums over runs of equal b, and per-step segmented sums over runs of equal
-// b) over the same pairs sorted by b.  The two instances together add the
-// same six targets as ROLE 0 with twice the integral work and several times
-// fewer atomic requests.
+// small s/p classes, so every quartet is evaluated twice: by the a-side
+// instance (ROLE 1: J(a,b), J(c,d), K(a,c), K(a,d)) over P lists sorted by a,
+// and by the b-side instance (ROLE 2: K(b,c), K(b,d), as register sums over
+// runs of equal c flushed by segmented sums over runs of equal b, and per-step
+// segmented sums over runs of equal b) over the same pairs sorted by b.  The
+// tile kernel (jk_tile.h) does the same in one pass and is faster; these run
+// where BQCset_row_split asks for them.
 #pragma once
 #include "jk_kernel.h"
 
-// Most roots whose table the row kernels stage in LDS
-#define BQC_RYS_LDS_MAX 4
 // Work counters per persistent launch: the item list is cut into this many
 // contiguous slices, one per XCD (workgroups are dispatched to the XCDs in
 // turn, so workgroup b runs on XCD b % 8)
@@ -181,21 +178,17 @@ struct ItemQueue {
 };
 
 // Work item: (task, chunk of 64 P pairs, first and end Q position).
-template <int LA, int LB, int LC, int LD, typename T, int ROLE = 0>
+template <int LA, int LB, int LC, int LD, int ROLE>
 __global__ void __launch_bounds__(256)
     jk_rows(const TaskDesc *__restrict__ tasks, const int4 *__restrict__ items, int nitems,
             int *ticket) {
     using C = Cls<LA, LB, LC, LD>;
     constexpr int NA = C::NFI, NB = C::NFJ, NC = C::NFK, ND = C::NFL;
     // Rys interpolation table of this class's root count staged in LDS
-    // (9, 21, 36, 53 KB for 1 to 4 roots) before any wave leaves
-    constexpr bool RYS_LDS = C::NR <= BQC_RYS_LDS_MAX;
-    constexpr int RYS_N = RYS_LDS ? rys_lds_size(C::NR) : 2;
-    __shared__ __align__(16) double rys_lds[RYS_N];
-    if constexpr (RYS_LDS) {
-        rys_stage<C::NR, 256>(rys_lds);
-        __syncthreads();
-    }
+    // (9, 21, 36 KB for 1 to 3 roots) before any wave leaves
+    __shared__ __align__(16) double rys_lds[rys_lds_size(C::NR)];
+    rys_stage<C::NR, 256>(rys_lds);
+    __syncthreads();
     const rys_lds_ptr rys_tab = (rys_lds_ptr)rys_lds;
     // per-wavefront staging of packed atomics
     constexpr int PK = row_pack_max<NA, NB, NC, ND>();
@@ -304,26 +297,20 @@ __global__ void __launch_bounds__(256)
                     active = active && ppos >= qpos;
                     if (ppos == qpos) norm *= 0.5;
                 }
-                T g[C::NF];
+                double g[C::NF];
                 if (active) {
                     // first Q primitive pair, marked wave-uniform so that the
                     // primitive loop reads its data with scalar loads
                     const int qq0 = __builtin_amdgcn_readfirstlane(tk.prim_q0 + qpos * tk.nprim_q);
                     const double rc[3] = {ubx[sc], uby[sc], ubz[sc]};
                     const double rd[3] = {ubx[sd], uby[sd], ubz[sd]};
-                    if constexpr (RYS_LDS)
-                        eri_block<LA, LB, LC, LD, T>(g, pd, pp0, tk.nprim_p,
-                                                     qq0, tk.nprim_q,
-                                                     norm, ra, rb, rc, rd, 0, rys_tab, p_first);
-                    else
-                        eri_block<LA, LB, LC, LD, T>(g, pd, pp0, tk.nprim_p,
-                                                     qq0, tk.nprim_q,
-                                                     norm, ra, rb, rc, rd, 0, nullptr, p_first);
+                    eri_block<LA, LB, LC, LD, double>(g, pd, pp0, tk.nprim_p, qq0, tk.nprim_q,
+                                                      norm, ra, rb, rc, rd, 0, rys_tab, p_first);
                 } else {
 #pragma unroll
-                    for (int n = 0; n < C::NF; ++n) g[n] = (T)0;
+                    for (int n = 0; n < C::NF; ++n) g[n] = 0;
                 }
-#define G(x, y, z, w) ((double)g[(((x) * NB + (y)) * NC + (z)) * ND + (w)])
+#define G(x, y, z, w) (g[(((x) * NB + (y)) * NC + (z)) * ND + (w)])
                 if (ROLE != 2 && VJ) {
                     // J(a,b) += g D(c,d)
 #pragma unroll
@@ -410,7 +397,7 @@ __global__ void __launch_bounds__(256)
                                 if (off[v] >= 0) atomic_add(VK + off[v], val[v]);
                         }
                     }
-                    // K(b,d): per lane (segmented over runs of equal b in the b-side role)
+                    // K(b,d): segmented over runs of equal b, added by the run tails
                     if constexpr (ROLE != 1) {
                         constexpr int NV = NB * ND;
                         double val[NV];
@@ -424,13 +411,8 @@ __global__ void __launch_bounds__(256)
                                 for (int x = 0; x < NA; ++x)
 #pragma unroll
                                     for (int z = 0; z < NC; ++z) s += G(x, y, z, w) * dac[x * NC + z];
-                                if constexpr (ROLE == 2) {
-                                    val[w * NB + y] = run_scan(s, lane, run_start);
-                                    off[w * NB + y] = tail && pvalid ? (d0 + w) * nao + b0 + y : -1;
-                                } else {
-                                    val[w * NB + y] = s;
-                                    off[w * NB + y] = active ? (d0 + w) * nao + b0 + y : -1;
-                                }
+                                val[w * NB + y] = run_scan(s, lane, run_start);
+                                off[w * NB + y] = tail && pvalid ? (d0 + w) * nao + b0 + y : -1;
                             }
                         if constexpr (pack_nv(NV) > 0) {
                             packed_atomic_add<NV>(VK, val, off, sv, so, lane);
@@ -473,16 +455,8 @@ __global__ void __launch_bounds__(256)
                         for (int z = 0; z < NC; ++z)
 #pragma unroll
                             for (int y = 0; y < NB; ++y) {
-                                if constexpr (ROLE == 2) {
-                                    val[z * NB + y] = run_scan(kbc[y * NC + z], lane, run_start);
-                                    off[z * NB + y] =
-                                        tail && pvalid ? (c0 + z) * nao + b0 + y : -1;
-                                } else {
-                                    val[z * NB + y] = kbc[y * NC + z];
-                                    off[z * NB + y] = pvalid && kbc[y * NC + z] != 0.0
-                                                          ? (c0 + z) * nao + b0 + y
-                                                          : -1;
-                                }
+                                val[z * NB + y] = run_scan(kbc[y * NC + z], lane, run_start);
+                                off[z * NB + y] = tail && pvalid ? (c0 + z) * nao + b0 + y : -1;
                                 kbc[y * NC + z] = 0.0;
                             }
                         if constexpr (pack_nv(NV) > 0) {
@@ -517,36 +491,18 @@ __global__ void __launch_bounds__(256)
 }
 
 typedef void (*RowKernel)(const TaskDesc *, const int4 *, int, int *);
-// [role][precision][bra pair id][ket pair id]: role 0 the single pass, roles
-// 1 and 2 the a-side and b-side passes of split classes (FP64 only), 3 the
-// tile kernel (FP64 only, jk_tile.h)
-typedef RowKernel RowKernelTable[4][2][BQC_NPAIRID][BQC_NPAIRID];
+// [role][bra pair id][ket pair id]: role 0 the tile kernel (jk_tile.h), roles
+// 1 and 2 the a-side and b-side passes of split classes.  FP64 only: mixed
+// builds run these classes in FP64 throughout.  Packed FP32 is off, so an FP32
+// operation costs an FP64 one, and a row's Q range cut in two by precision
+// pays its set-up and flushes twice.  FP64 tile kernel against FP64 + FP32
+// kernels of the bins (ms): 40 waters cc-pVTZ (dp|pp) 28.5 / 68.9, (ds|ps) 31.2
+// / 41.3, (dp|dp) 39.1 / 47.7, (dp|ss) 20.9 / 27.6, (fs|dp) 19.1 / 31.0; only
+// (dd|ds) and (dd|pp) of 64 dense waters cc-pVDZ were better split, 2.7 / 1.5
+// and 3.3 / 2.4.
+typedef RowKernel RowKernelTable[3][BQC_NPAIRID][BQC_NPAIRID];
 
-// Classes digested with the wavefront-stationary kernel, per precision.
-// Up to 108 Cartesian components the FP64 block and the lane accumulators
-// fit the 512 registers of one wave per SIMD (with small spills), and this
-// kernel beats the wavefront-per-quartet one by ~3x (measured on (dp|ds));
-// at 162 the spills make it slower than that kernel.  The FP32 instance has
-// the same limit: at 162-216 components (2-3 KB of scratch per lane) it ran
-// at 1.2-1.4 TFLOP/s against 2.4-3.5 for the wavefront-per-quartet kernel.
-template <int LA, int LB, int LC, int LD, typename T>
-constexpr bool use_rows() {
-    return Cls<LA, LB, LC, LD>::NF <= 108;
-}
-
-// Row classes with an FP32 instance (used by mixed precision).  The others
-// are bound by atomic requests, which FP32 integrals do not reduce, while
-// splitting a row's Q range by precision adds a flush of its accumulators:
-// with every row class split, 64 H2O cc-pVDZ took 168 ms against 158 ms in
-// FP64; on 128 H2O cc-pVTZ these six gained 7-105 ms each and the rest
-// -3..+2 ms.  Mixed builds run the quartets of the others in FP64.
-template <int LA, int LB, int LC, int LD>
-constexpr bool row_fp32() {
-    constexpr int c = LA * 1000 + LB * 100 + LC * 10 + LD;
-    return c == 2010 || c == 2100 || c == 2120 || c == 2210 || c == 3020 || c == 3110;
-}
-
-// Row classes compiled with the a-side / b-side pair as well: the small s/p
+// Classes compiled with the a-side / b-side pair as well: the small s/p
 // classes, whose time goes to atomic requests rather than arithmetic.  Whether
 // a build uses the pair is chosen per class at run time (BQCset_row_split).
 template <int LA, int LB, int LC, int LD>

@@ -445,7 +445,10 @@ template <int LA, int LB, int LC, int LD>
 static void reg_wave(WaveKernelTable &tab) {
     if constexpr (use_wave<LA, LB, LC, LD>()) {
         tab[0][LA * (LA + 1) / 2 + LB][LC * (LC + 1) / 2 + LD] = jk_wave<LA, LB, LC, LD, double>;
-        tab[1][LA * (LA + 1) / 2 + LB][LC * (LC + 1) / 2 + LD] = jk_wave<LA, LB, LC, LD, float>;
+        // mixed builds run the tile classes in FP64 (RowKernelTable)
+        if constexpr (!use_tile<LA, LB, LC, LD>())
+            tab[1][LA * (LA + 1) / 2 + LB][LC * (LC + 1) / 2 + LD] =
+                jk_wave<LA, LB, LC, LD, float>;
     }
 }
 
