@@ -128,8 +128,9 @@ void BQCdel_basis_prod_clone(BasisProdCache **pbp);
  * precision: 0 = FP64
  * throughout; 1 = mixed: a quartet is evaluated in FP32 (Rys roots and
  * weights, prefactors and all J/K accumulation stay FP64) when the upper
- * bound q_P q_Q dmax of its Schwarz bins, taken over the 64 pairs sharing a
- * wavefront, falls below fp32_cut.  log_q (host, one per pair, plan order)
+ * bound q_P q_Q dmax of its Schwarz bins falls below fp32_cut and its class
+ * gains by it: the classes of the wave kernels.  The others (up to 81
+ * components, and larger ones with a tile kernel) stay in FP64.  log_q (host, one per pair, plan order)
  * gives log q; task_dmax (host, one per task) the task's density bound.
  * log_q is used for this split only (the bins come from task_bins), so it
  * may hold the unclipped log q of every pair.
@@ -188,8 +189,9 @@ void BQCgraph_destroy(void *graph);
  * on the molecule's Cartesian AO count (read off the autotuner on MI355X:
  * rows / rows of classes above 81 components / waves 128 / 128 / 32 below
  * 2048 AOs (32 for (ss|ss), 16 for (pp|pp)), 64 / 64 / 32 from 2048,
- * 256 / 128 / 64 from 8192; 64 waters cc-pVDZ, 2624 AOs, ran 6 ms faster on
- * 64 than on 256 Q pairs per row item).  Precedence when a build is
+ * 256 / 128 / 64 from 8192).  These are the values that BQCget_tile reports;
+ * where none is set, the tile kernels take items of up to 256 Q pairs, and
+ * launches with little work shorter ones.  Precedence when a build is
  * planned: per-class setting,
  * all-class setting, default.  Process-wide; used by the tile autotuner;
  * not to be called while another thread plans a build.
