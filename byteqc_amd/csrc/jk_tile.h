@@ -66,6 +66,23 @@ struct TileCls {
     // with two and 95 spilled registers (12 molecules def2-SVP); (ps|ss) 27.6
     // with two, 24.2 with three.
     static constexpr int WAVES = NF <= 3 ? 3 : (NF <= 27 ? 2 : 1);
+    // Values a lane holds beside the integrals' temporaries: D and J of (a,b),
+    // the accumulators and densities of a c-run, D of d, J(c,d), the block.
+    // Where they take over 0.6 of the registers (512 / WAVES of 32 bits), the
+    // accumulators and densities were spilled and reloaded around every
+    // block, to scratch far beyond the L2: (pp|ps) moved 35 GB in 7.9 ms for
+    // 64 waters cc-pVDZ.  RELOAD: the densities D(b,c), D(a,c) are read at
+    // every step instead of once per c-run.  DIRECT: K(a,c), K(b,c) are added
+    // to the LDS block at every step instead of accumulating over the run,
+    // which pays at two waves where the additions are fewer than the
+    // components.  Held / RELOAD / DIRECT too (ms, 12 molecules def2-SVP):
+    // (pp|ps) 16.0 / 14.4 / 12.6, (dp|ss) 4.9 / 4.4 / 4.1, (ds|ps) 9.3 / 7.9 /
+    // 8.4, (pp|pp) 6.4 / 5.9 / 6.6, (dp|ps) 8.3 / 8.1 / 7.9; below the line
+    // (ds|pp) 4.7 / 4.9 / 4.8, (ds|ds) 2.1 / 2.1 / 2.3.
+    static constexpr int LIVE =
+        2 * NA * NB + 2 * (NA + NB) * NC + (NA + NB) * ND + NC * ND + NF;
+    static constexpr bool RELOAD = LIVE * WAVES > 153;
+    static constexpr bool DIRECT = RELOAD && WAVES == 2 && (NA + NB) * NC < NF;
     // doubles of LDS per wavefront for the block of K: what WAVES workgroups
     // per CU leave of 160 KB after the Rys table and the row and column lists
     static constexpr int CAP = (163840 / WAVES - rys_lds_size(C::NR) * 8 -
@@ -298,6 +315,15 @@ __global__ void __launch_bounds__(256, (TileCls<LA, LB, LC, LD>::WAVES))
                 for (int k = 0; k < NA * NC; ++k) kac[k] = dac[k] = 0.0;
 #pragma unroll
                 for (int k = 0; k < NB * NC; ++k) kbc[k] = dbc[k] = 0.0;
+                auto load_c = [&](int c0) {
+#pragma unroll
+                    for (int z = 0; z < NC; ++z) {
+#pragma unroll
+                        for (int y = 0; y < NB; ++y) dbc[y * NC + z] = D[(c0 + z) * nao + b0 + y];
+#pragma unroll
+                        for (int x = 0; x < NA; ++x) dac[x * NC + z] = D[(c0 + z) * nao + a0 + x];
+                    }
+                };
                 auto flush_c = [&](int col) {
 #pragma unroll
                     for (int z = 0; z < NC; ++z) {
@@ -340,17 +366,9 @@ __global__ void __launch_bounds__(256, (TileCls<LA, LB, LC, LD>::WAVES))
                             for (int x = 0; x < NA; ++x) dad[x * ND + w] = D[(d0 + w) * nao + a0 + x];
                         }
                         if (colc != ccol) {
-                            if (ccol >= 0) flush_c(ccol);
+                            if (!TC::DIRECT && ccol >= 0) flush_c(ccol);
                             ccol = colc;
-#pragma unroll
-                            for (int z = 0; z < NC; ++z) {
-#pragma unroll
-                                for (int y = 0; y < NB; ++y)
-                                    dbc[y * NC + z] = D[(c0 + z) * nao + b0 + y];
-#pragma unroll
-                                for (int x = 0; x < NA; ++x)
-                                    dac[x * NC + z] = D[(c0 + z) * nao + a0 + x];
-                            }
+                            if (!TC::RELOAD) load_c(c0);
                         }
                     }
                     double g[TC::NF];
@@ -389,6 +407,7 @@ __global__ void __launch_bounds__(256, (TileCls<LA, LB, LC, LD>::WAVES))
                             }
                     }
                     if (do_k) {
+                        if (TC::RELOAD) load_c(c0);
 #pragma unroll
                         for (int x = 0; x < NA; ++x)
 #pragma unroll
@@ -401,6 +420,7 @@ __global__ void __launch_bounds__(256, (TileCls<LA, LB, LC, LD>::WAVES))
                                         kac[x * NC + z] += v * dbd[y * ND + w];
                                         kbc[y * NC + z] += v * dad[x * ND + w];
                                     }
+                        if (TC::DIRECT) flush_c(colc);
 #pragma unroll
                         for (int w = 0; w < ND; ++w) {
 #pragma unroll
@@ -426,7 +446,7 @@ __global__ void __launch_bounds__(256, (TileCls<LA, LB, LC, LD>::WAVES))
 #undef G
                 }
                 if (do_k) {
-                    if (ccol >= 0) flush_c(ccol);
+                    if (!TC::DIRECT && ccol >= 0) flush_c(ccol);
                     wave_sync();
                     // consecutive rows are often consecutive functions, so an
                     // instruction's lanes share 64-byte segments
