@@ -19,7 +19,8 @@
 // jk_tile (ms): 64 waters cc-pVDZ (ps|ps) 18.4 -> 8.6, (ss|ss) 14.8 -> 8.9,
 // (ps|ss) 17.4 -> 14.2, all classes 110.6 -> 86.7; 24 waters cc-pVTZ (ps|ss)
 // 7.9 -> 3.0, (fs|ss) 3.2 -> 1.0, all classes 172 -> 138; 12 molecules
-// def2-SVP all classes 227 -> 187.  What is left of (ps|ss) at 64 waters, from
+// def2-SVP all classes 227 -> 187 (86.7, 138 and 187 are 73.9, 100.6 and 141.8
+// with the steps noted below).  What is left of (ps|ss) at 64 waters, from
 // variants that skip a part: integrals 4 ms, the block's atomics 2.7, J 1.8,
 // density gathers 1.2, item set-up 4.3; in batches of def2-SVP molecules the
 // integrals of the contracted shells are 3/4 of the time.
@@ -63,8 +64,8 @@ struct TileCls {
     static constexpr int NF = NA * NB * NC * ND;
     // resident wavefronts per SIMD, and so workgroups per CU: what registers
     // allow with few spills.  (pp|ps) runs 20.3 ms with one and no spills, 15.8
-    // with two and 95 spilled registers (12 molecules def2-SVP); (ps|ss) 27.6
-    // with two, 24.2 with three.
+    // with two and 95 spilled registers, 12.6 with what RELOAD and DIRECT below
+    // spare (12 molecules def2-SVP); (ps|ss) 27.6 with two, 24.2 with three.
     static constexpr int WAVES = NF <= 3 ? 3 : (NF <= 27 ? 2 : 1);
     // Values a lane holds beside the integrals' temporaries: D and J of (a,b),
     // the accumulators and densities of a c-run, D of d, J(c,d), the block.
