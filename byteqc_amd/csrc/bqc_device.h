@@ -15,17 +15,12 @@
 
 #define BQC_RYS_QUAL static __device__
 #include "rys_table.inc"
+#include "bqc_math.h"
 
 namespace bqc {
 
 constexpr int ncart(int l) { return (l + 1) * (l + 2) / 2; }
 constexpr int nroots_of(int li, int lj, int lk, int ll) { return (li + lj + lk + ll) / 2 + 1; }
-constexpr int rys_xbig(int n) { return 36 + 8 * n; }
-constexpr int rys_offset(int n) {
-    int off = 0;
-    for (int m = 1; m < n; ++m) off += rys_xbig(m) * 2 * m * (BQC_RYS_DEG + 1);
-    return off;
-}
 
 // Cartesian exponents of component c of a shell with angular momentum l
 // (order: lx from l down to 0, then ly from l-lx down to 0).
@@ -48,24 +43,6 @@ __host__ __device__ constexpr int cart_z(int l, int c) { return l - cart_x(l, c)
 // 2*pi^(5/2): prefactor of the Rys integrals (cuobc/lib/gint/g2e.c:41)
 constexpr double TWO_PI_52 = 34.98683665524972497;
 
-// 1/x and 1/sqrt(x) of positive normal numbers to about one unit in the last
-// place: the hardware estimate (24 bits) and one third-order step, 4 and 6
-// instructions; the compiler's division takes 11 and its square root 14,
-// mostly for denormals, infinities and correct rounding.
-__device__ __forceinline__ double fast_rcp(double x) {
-    const double r = __builtin_amdgcn_rcp(x);
-    const double e = fma(-x, r, 1.0);
-    return fma(r, fma(e, e, e), r);
-}
-__device__ __forceinline__ double fast_rsqrt(double x) {
-    const double r = __builtin_amdgcn_rsq(x);
-    const double e = fma(-x * r, r, 1.0);
-    return fma(r * e, fma(e, 0.375, 0.5), r);
-}
-
-// Number of doubles of the interpolation table of N roots.
-constexpr int rys_table_size(int n) { return rys_xbig(n) * 2 * n * (BQC_RYS_DEG + 1); }
-
 // Nodes and weights for x >= XBIG(N), the Gauss-Hermite limit.
 template <int N>
 __device__ __forceinline__ void rys_roots_far(double x, double *__restrict__ u,
@@ -74,57 +51,23 @@ __device__ __forceinline__ void rys_roots_far(double x, double *__restrict__ u,
 #pragma unroll
     for (int i = 0; i < N; ++i) {
         const double h = BQC_RYS_HERM_S[(N - 1) * BQC_RYS_NMAX + i];
-        u[i] = h * fast_rcp(x - h);
+        u[i] = fast_div(h, x - h);
         w[i] = BQC_RYS_HERM_W[(N - 1) * BQC_RYS_NMAX + i] * sq;
     }
 }
 
-// Copy of the N-root part of the table in LDS, in powers of y instead of
-// Chebyshev polynomials (one FMA per term where Clenshaw's rule takes two
-// operations).  The lanes of a wavefront read 16 bytes each from rows of
-// different intervals; two doubles of padding make the row length an odd
-// number of 16-byte units, so that rows start in all 16 groups of LDS banks
-// (rows of 24 N doubles start in four groups for one root, in two for two).
-constexpr int rys_lds_stride(int n) { return 2 * n * (BQC_RYS_DEG + 1) + 2; }
-constexpr int rys_lds_size(int n) { return rys_xbig(n) * rys_lds_stride(n); }
-
-// Coefficient of y^k in the Chebyshev polynomial T_n(y): t[n][k].
-struct ChebTable {
-    double t[BQC_RYS_DEG + 1][BQC_RYS_DEG + 1];
-    constexpr ChebTable() : t() {
-        for (int n = 0; n <= BQC_RYS_DEG; ++n)
-            for (int k = 0; k <= BQC_RYS_DEG; ++k)
-                t[n][k] = n < 2 ? (n == k ? 1.0 : 0.0)
-                                : (k > 0 ? 2.0 * t[n - 1][k - 1] : 0.0) - t[n - 2][k];
-    }
-};
-
-// Fills tab (rys_lds_size(N) doubles of LDS) with all lanes of a workgroup;
-// the caller synchronises.
+// Fills tab (rys_lds_size(N) doubles of LDS: a row of powers per interval)
+// with all lanes of a workgroup; the caller synchronises.
 template <int N, int NTHR>
 __device__ __forceinline__ void rys_stage(double *tab) {
-    constexpr ChebTable ch{};
     const double *src = BQC_RYS_COEF + rys_offset(N);
-    for (int i = threadIdx.x; i < rys_xbig(N) * 2 * N; i += NTHR) {
-        const double *c = src + i * (BQC_RYS_DEG + 1);
-        double *m = tab + (i / (2 * N)) * rys_lds_stride(N) + (i % (2 * N)) * (BQC_RYS_DEG + 1);
-        double v[BQC_RYS_DEG + 1];
-#pragma unroll
-        for (int n = 0; n <= BQC_RYS_DEG; ++n) v[n] = c[n];
-#pragma unroll
-        for (int k = 0; k <= BQC_RYS_DEG; ++k) {
-            double s = 0.0;
-#pragma unroll
-            for (int n = BQC_RYS_DEG; n >= k; --n)
-                if ((n - k) % 2 == 0) s = fma(ch.t[n][k], v[n], s);
-            m[k] = s;
-        }
-    }
+    for (int i = threadIdx.x; i < rys_xbig(N) * N; i += NTHR)
+        rys_stage_root<N>(src + i / N * (2 * N * (BQC_RYS_DEG + 1)),
+                          tab + i / N * rys_lds_stride(N), i % N);
 }
 
 // Nodes u_i = t_i^2 / (1 - t_i^2) and weights of the N-point Rys rule for
 // argument x, from the table in LDS (rys_stage).
-typedef double rys_pair __attribute__((ext_vector_type(2)));
 typedef const __attribute__((address_space(3))) rys_pair *rys_lds_ptr;
 template <int N>
 __device__ __forceinline__ void rys_roots(double x, double *__restrict__ u,
@@ -133,25 +76,8 @@ __device__ __forceinline__ void rys_roots(double x, double *__restrict__ u,
         rys_roots_far<N>(x, u, w);
         return;
     }
-    const double y = fma(2.0, __builtin_amdgcn_fract(x), -1.0), y2 = y * y;
-    const rys_lds_ptr c = tab + (int)x * (rys_lds_stride(N) / 2);
-    // even and odd powers of all functions side by side: 4 N chains of 5
-    // dependent operations instead of 2 N of 11
-    constexpr int H = (BQC_RYS_DEG + 1) / 2;
-    static_assert(BQC_RYS_DEG % 2 == 1, "coefficients are read in pairs");
-    rys_pair v[2 * N];
-#pragma unroll
-    for (int f = 0; f < 2 * N; ++f) v[f] = c[f * H + H - 1];
-#pragma unroll
-    for (int j = H - 2; j >= 0; --j)
-#pragma unroll
-        for (int f = 0; f < 2 * N; ++f) {
-            const rys_pair p = c[f * H + j];
-            v[f].x = fma(y2, v[f].x, p.x);
-            v[f].y = fma(y2, v[f].y, p.y);
-        }
-#pragma unroll
-    for (int f = 0; f < 2 * N; ++f) (f < N ? u[f] : w[f - N]) = fma(y, v[f].y, v[f].x);
+    const double y = fma(2.0, __builtin_amdgcn_fract(x), -1.0);
+    rys_from_row<N>(y, tab + (int)x * (rys_lds_stride(N) / 2), u, w);
 }
 
 // The same from the N-root part of the table in global memory.
@@ -197,7 +123,7 @@ __device__ __forceinline__ void rys_root_one(double x, int r, double &u, double 
     static_assert(N >= 1 && N <= BQC_RYS_NMAX, "unsupported number of roots");
     if (x >= (double)rys_xbig(N)) {
         const double h = BQC_RYS_HERM_S[(N - 1) * BQC_RYS_NMAX + r];
-        u = h * fast_rcp(x - h);
+        u = fast_div(h, x - h);
         w = BQC_RYS_HERM_W[(N - 1) * BQC_RYS_NMAX + r] * fast_rsqrt(x);
         return;
     }

@@ -125,10 +125,11 @@ __device__ __forceinline__ void atomic_add(gdouble *p, double v) {
 // this class's root count in LDS (rys_stage).
 // A primitive quartet of (ps|ss) is some 95 FP64 instructions in dependent
 // chains, and the wavefronts that fit beside the accumulators do not hide the
-// latencies: so the Q data of the next one are loaded ahead, divisions and
-// square roots are 4-6 instructions, and the Rys polynomials run as parallel
-// chains (12 molecules def2-SVP, all classes: 215 -> 202 ms from the short
-// reciprocals, 187 -> 181 from the loads ahead and the parallel chains).  The
+// latencies: so the Q data of the next one are loaded ahead, reciprocals and
+// the factors of the quartet are short sequences (bqc_math.h), and the Rys
+// polynomials run as parallel chains (12 molecules def2-SVP, all classes: 215
+// -> 202 ms from the short reciprocals, 187 -> 181 from the loads ahead and the
+// parallel chains; of which 5 ms go into rounding them like quotients).  The
 // P pairs of a wavefront's lanes lie apart: their records take 64 lines of L1
 // per primitive instead of 320 (181 -> 175 ms, 40 waters mixed 52.5 -> 50.1).
 // FLAT: all loops unrolled (needs a compile-time x0), so that the block stays
@@ -195,13 +196,13 @@ __device__ __forceinline__ void eri_block(T *__restrict__ gout, const PairData &
             const double pq[3] = {P[0] - Q[0], P[1] - Q[1], P[2] - Q[2]};
             const double aijkl = aij + akl;
             const double a1 = aij * akl;
-            const double rs = fast_rsqrt(aijkl);
-            const double a0 = a1 * (rs * rs);
+            const QuartetScale qs(a1, aijkl);
+            const double a0 = qs.a0;
             const double x = a0 * (pq[0] * pq[0] + pq[1] * pq[1] + pq[2] * pq[2]);
             double u[NR], w[NR];
             if constexpr (std::is_same<RysPtr, std::nullptr_t>::value) rys_roots<NR>(x, u, w);
             else rys_roots<NR>(x, u, w, rys_tab);
-            const double fac = eij * ekl * rs * fast_rcp(a1);
+            const double fac = eij * ekl * qs.scale;
 #pragma unroll
             for (int r = 0; r < NR; ++r) {
                 const double u2 = a0 * u[r];

@@ -255,7 +255,8 @@ __global__ void __launch_bounds__(64, (wave_min_waves<LA, LB, LC, LD>()))
                         const double Q[3] = {ux12[qq], uy12[qq], uz12[qq]};
                         const double pq[3] = {P[0] - Q[0], P[1] - Q[1], P[2] - Q[2]};
                         const double aijkl = aij + akl, a1 = aij * akl;
-                        const double rs = fast_rsqrt(aijkl), a0q = a1 * (rs * rs);
+                        const QuartetScale qs(a1, aijkl);
+                        const double a0q = qs.a0;
                         const double x = a0q * (pq[0] * pq[0] + pq[1] * pq[1] + pq[2] * pq[2]);
                         // phase A: one (direction, root) table per lane
                         if (lane < 3 * NR) {
@@ -268,7 +269,7 @@ __global__ void __launch_bounds__(64, (wave_min_waves<LA, LB, LC, LD>()))
                             const double b10 = b00 + tmp4 * akl;
                             const double b01 = b00 + tmp4 * aij;
                             const double seed = d == 0 ? norm
-                                                : (d == 1 ? eij * ekl * rs * fast_rcp(a1) : wr);
+                                                : (d == 1 ? eij * ekl * qs.scale : wr);
                             const double Pd = d == 0 ? P[0] : (d == 1 ? P[1] : P[2]);
                             const double Qd = d == 0 ? Q[0] : (d == 1 ? Q[1] : Q[2]);
                             const double Ad = d == 0 ? ra[0] : (d == 1 ? ra[1] : ra[2]);
