@@ -224,6 +224,15 @@ int BQCset_row_split(int cls, int on);
  * counterpart in the reference.  Returns 0 ok, 1 bad argument. */
 int BQCset_prim_records(BasisProdCache *bpcache, const double *records);
 
+/* Side streams that the library holds.  BQCbuild_jk and BQCbuild_jk_batch run
+ * their launches next to each other on the caller's stream and a device's set
+ * of three side streams, which is made on first use, kept, and lent to one
+ * build at a time: a build that finds it in use by another stream's launches
+ * (or is made into a stream capture) runs on its own stream alone.  Whatever
+ * follows a build on its stream sees all its launches.  Returns three per
+ * device with builds so far, whatever the number of streams. */
+int BQCside_streams(void);
+
 /* Launch shape of the row kernels.  Persistent grids have as many
  * workgroups as fit on the device at once, each wavefront pulling work items
  * from a counter in the build's work list until it is exhausted; the other
