@@ -1869,6 +1869,13 @@ int BQCget_tile(int kind, int cls, int prec, int nao) {
     return tile_for(kind, cls, prec, nao);
 }
 
+int BQCget_set_tile(int kind, int cls, int prec) {
+    if (kind != 1 && kind != 4) return -1;
+    bool fixed;
+    const int ck = tile_for(kind, cls, prec, 0, &fixed);
+    return fixed ? ck : 0;
+}
+
 void BQCprofile_enable(int on) {
     g_prof = on != 0;
 }

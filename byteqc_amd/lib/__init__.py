@@ -44,6 +44,7 @@ _SIGNATURES = {
     'BQCgraph_destroy': (None, [c_void_p]),
     'BQCset_tile': (c_int, [c_int, c_int, c_int, c_int]),
     'BQCget_tile': (c_int, [c_int, c_int, c_int, c_int]),
+    'BQCget_set_tile': (c_int, [c_int, c_int, c_int]),
     'BQCside_streams': (c_int, []),
     'BQCset_prim_records': (c_int, [c_void_p, c_void_p]),
     'BQCset_launch_mode': (c_int, [c_int]),

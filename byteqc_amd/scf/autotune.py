@@ -8,13 +8,14 @@ work items (better fill of the 256 CUs for classes with few pairs) at the
 cost of more flushes of the lane accumulators (J(a,b), K(a,c), K(b,c));
 a large ck gives fewer flushes and fewer items.
 
-``tune(run)`` times every candidate with the library's per-launch HIP-event
-records (one launch per class, kind and precision per build), keeps the
-fastest ck per (kind, class, precision) and installs it with
-``BQCset_tile``.  Without tuning the library uses default tiles chosen by
-molecule size (large molecules want long Q ranges per item, batches of
-small ones short), measured the same way over the benchmark workloads.  Any tile gives the same quartet set and the same sums
-(only the order of floating-point accumulation differs).
+Without a setting the library cuts items by the load of each launch, up to a
+largest range per kernel kind; a tile that is set replaces that rule by one
+length.  ``tune(run)`` times the rule and every candidate with the library's
+per-launch HIP-event records (one launch per class, kind and precision per
+build) and sets a tile with ``BQCset_tile`` only for the (kind, class,
+precision) in which one is faster than the rule.  Any tile gives the same
+quartet set and the same sums (only the order of floating-point accumulation
+differs).
 
 The reference has fixed launch shapes per class (nr_jk_driver.cu:46-225).
 """
@@ -31,6 +32,8 @@ from byteqc_amd.scf import hf
 ROWS, WAVE = 1, 4
 CANDIDATES = {ROWS: (16, 32, 64, 128, 256), WAVE: (8, 16, 32, 64, 128)}
 DEFAULTS = {ROWS: 64, WAVE: 32}     # reference point for a table without recorded defaults
+RULE = 0       # in a table: items cut by load, no tile set
+MARGIN = 0.02  # a tile has to beat the rule by this share, more than two runs differ
 
 
 def reset():
@@ -39,9 +42,11 @@ def reset():
 
 
 def current_tile(kind, cls, prec, nao):
-    """Tile a build of a molecule with nao Cartesian AOs planned now uses for
-    (kind, cls, prec): a tuned tile if one is installed, else the default."""
-    return int(load_library().BQCget_tile(int(kind), int(cls), int(prec), int(nao)))
+    """Tile that builds planned now use for (kind, cls, prec): the one that is
+    set for the class or for the kind, else RULE (0): items are cut by the load
+    of each launch.  nao (Cartesian AOs of the molecule) does not matter for
+    either."""
+    return int(load_library().BQCget_set_tile(int(kind), int(cls), int(prec)))
 
 
 def _timed(run, reps):
@@ -58,52 +63,68 @@ def _timed(run, reps):
     return hf.profile_read()
 
 
+def _class_times(run, reps):
+    """{(kind, cls, prec): ms per build} with the tiles as they are."""
+    agg = defaultdict(float)
+    for r in _timed(run, reps):
+        # kind: 1 row / 4 wavefront kernel, + 2 FP32, + 8 b-side pass of a
+        # split class (both passes of a class share its tile), + 16 tile kernel
+        kind = r['kind'] & ~26
+        if kind in (ROWS, WAVE):
+            agg[(kind, r['cls'], (r['kind'] >> 1) & 1)] += r['ms'] / reps
+    return agg
+
+
 def tune(run, candidates=None, reps=1, nao=0):
     """Tune tiles for the builds done by ``run()`` (one eager J/K build per
     call, any number of molecules; nao: Cartesian AO count of the largest,
-    which picks the default tiles recorded as 'builtin').  Returns
+    which picks the size band recorded as 'builtin').  Returns
     {(kind, cls, prec): {'ck': best, 'ms': {ck: ms per build}, 'builtin':
-    default ck}} and leaves the best tiles installed."""
+    size band's ck}}, where ck RULE stands for items cut by load, and leaves
+    the best tiles set."""
     lib = load_library()
     candidates = candidates or CANDIDATES
     reset()
     times = defaultdict(dict)
+    for key, ms in _class_times(run, reps).items():
+        times[key][RULE] = ms
     for kind, cks in candidates.items():
         for ck in cks:
             if lib.BQCset_tile(kind, -1, 0, int(ck)):
                 raise ValueError(f'bad tile {ck}')
-            agg = defaultdict(float)
-            for r in _timed(run, reps):
-                # kind: 1 row / 4 wavefront kernel, + 2 FP32, + 8 b-side pass,
-                # + 16 tile kernel
-                # of a split class (both passes of a class share its tile)
-                if (r['kind'] & ~26) != kind:
-                    continue
-                agg[(r['cls'], (r['kind'] >> 1) & 1)] += r['ms']
-            for (cls, prec), ms in agg.items():
-                times[(kind, cls, prec)][int(ck)] = ms / reps
+            for key, ms in _class_times(run, reps).items():
+                # a class that changes its kernel kind between the runs has
+                # no time of the rule to compare with
+                if key[0] == kind and RULE in times[key]:
+                    times[key][int(ck)] = ms
         reset()
     table = {}
     for key, per in times.items():
+        if RULE not in per:
+            continue
         best = min(per, key=per.get)
-        table[key] = {'ck': best, 'ms': per, 'builtin': current_tile(*key, nao)}  # after reset()
+        if per[best] > (1 - MARGIN) * per[RULE]:
+            best = RULE
+        table[key] = {'ck': best, 'ms': per, 'builtin': int(lib.BQCget_tile(*key, int(nao)))}
     install(table)
     return table
 
 
 def install(table):
-    """Install a tuned table (as returned by ``tune`` or ``load``)."""
+    """Set the tiles of a tuned table (as returned by ``tune`` or ``load``)."""
     lib = load_library()
     reset()
     for (kind, cls, prec), rec in table.items():
-        if lib.BQCset_tile(int(kind), int(cls), int(prec), int(rec['ck'])):
+        if rec['ck'] != RULE and lib.BQCset_tile(int(kind), int(cls), int(prec), int(rec['ck'])):
             raise ValueError(f'bad tile entry {(kind, cls, prec)}: {rec}')
 
 
 def gain(table):
-    """(ms per build with the default tiles, ms with tuned tiles) over the
-    table."""
-    base = sum(rec['ms'].get(rec.get('builtin', DEFAULTS[k]), min(rec['ms'].values()))
+    """(ms per build with items cut by load, ms with tuned tiles) over the
+    table; a table saved without times of the rule counts the size band's
+    tile in its place."""
+    base = sum(rec['ms'].get(RULE, rec['ms'].get(rec.get('builtin', DEFAULTS[k]),
+                                                 min(rec['ms'].values())))
                for (k, _, _), rec in table.items())
     tuned = sum(rec['ms'][rec['ck']] for rec in table.values())
     return base, tuned

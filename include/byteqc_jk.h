@@ -185,19 +185,23 @@ void BQCgraph_destroy(void *graph);
 /* Q pairs per work item of the row kernels (kind 1) or wave kernels
  * (kind 4), for class code cls (li*1000+lj*100+lk*10+ll as evaluated) and
  * precision prec (0 FP64, 1 FP32), or for all classes of the kind (cls < 0);
- * kind 0 clears these settings and restores the default tiles, which depend
- * on the molecule's Cartesian AO count (read off the autotuner on MI355X:
- * rows / rows of classes above 81 components / waves 128 / 128 / 32 below
- * 2048 AOs (32 for (ss|ss), 16 for (pp|pp)), 64 / 64 / 32 from 2048,
- * 256 / 128 / 64 from 8192).  These are the values that BQCget_tile reports;
- * where none is set, the tile kernels take items of up to 256 Q pairs, and
- * launches with little work shorter ones.  Precedence when a build is
- * planned: per-class setting,
- * all-class setting, default.  Process-wide; used by the tile autotuner;
- * not to be called while another thread plans a build.
+ * kind 0 clears these settings.  Where no tile is set, items are cut by the
+ * load of each launch, up to 256 Q pairs for the tile kernels and up to the
+ * size band that BQCget_tile reports for the others; a tile that is set
+ * replaces that rule by one length.  Bands by the molecule's Cartesian AO
+ * count (read off the autotuner on MI355X): rows / rows of classes above 81
+ * components / waves 128 / 128 / 32 below 2048 AOs (32 for (ss|ss), 16 for
+ * (pp|pp)), 64 / 64 / 32 from 2048, 256 / 128 / 64 from 8192.  Precedence when
+ * a build is planned: per-class setting, all-class setting, rule.
+ * Process-wide; used by the tile autotuner; not to be called while another
+ * thread plans a build.
  * No counterpart in the reference (its launch shapes are fixed per class,
  * nr_jk_driver.cu:46-225).  Returns 0 ok, 1 bad argument. */
 int BQCset_tile(int kind, int cls, int prec, int ck);
+
+/* The tile that is set for a class (per class or for all classes of the
+ * kind), or 0 where items are cut by load; -1 for another kind than 1 or 4. */
+int BQCget_set_tile(int kind, int cls, int prec);
 
 /* Whether the row-kernel class cls (code li*1000+lj*100+lk*10+ll as
  * evaluated; -1: all classes, clearing per-class settings) runs as two
