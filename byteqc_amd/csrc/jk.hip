@@ -422,8 +422,6 @@ static PairData make_pair_data(const BasisProdCache *bp) {
 // A BuildPlan collects the tasks of one or many molecules; items are grouped
 // by kernel so that every (class, precision, kernel kind) is one launch.
 // ---------------------------------------------------------------------------
-#define BQC_WAVE_CK 32
-
 #define BQC_CK_ROWS_DEFAULT 64
 #define BQC_CK_WAVE_DEFAULT 32
 static int g_ck_rows = BQC_CK_ROWS_DEFAULT;  // Q pairs per row-kernel item
@@ -616,30 +614,6 @@ static bool is_tile(RowKernel k) {
     return false;
 }
 
-// Kernels of a task per precision: the tile kernel of the class when there is
-// one within the scratch and LDS limits, else the wave kernels.  False if
-// there is neither (the generic kernels take the task).  *log_cut: the
-// precision rule, with every quartet in FP64 where the class has a tile kernel
-// or no FP32 instance (FP64 code for k[1] then, with no items).
-static bool pick_kernels(const TaskCtx &c, RowKernel (&k)[2], int (&wv)[2], double *log_cut) {
-    auto usable = [&](const auto &t) {
-        const RowKernel r = c.swap ? t[c.pkl][c.pij] : t[c.pij][c.pkl];
-        return r && scratch_ok((const void *)r) ? r : nullptr;
-    };
-    *log_cut = c.log_cut;
-    k[0] = usable(g_rows[0]);
-    wv[0] = !k[0];
-    if (!k[0]) k[0] = usable(g_waves[0]);
-    if (!k[0]) return false;
-    k[1] = wv[0] ? usable(g_waves[1]) : nullptr;
-    wv[1] = wv[0];
-    if (!k[1]) {
-        k[1] = k[0];
-        *log_cut = -1e300;
-    }
-    return true;
-}
-
 // First Q bin of P bin s whose quartets run in FP32 (nbins - s if none).
 static int fp32_split(const TaskCtx &c, int cp_p, int cp_q, const int *pbins, const int *qbins,
                       int s, double log_cut) {
@@ -649,17 +623,61 @@ static int fp32_split(const TaskCtx &c, int cp_p, int cp_q, const int *pbins, co
     return c.nbins - s;
 }
 
-// Work of the launches of a build, one entry per evaluated class and
-// precision, in primitive-quartet steps of a wavefront.  A step of a task
-// costs its primitive quartets plus BQC_STEP_BASE for the digestion.
+// Work of the launches of a build, one entry per evaluated class: the kernels
+// within the scratch and LDS limits, the wavefronts of each that fit on the
+// device, and the work per precision in primitive-quartet steps of a
+// wavefront.  A step of a task costs its primitive quartets plus BQC_STEP_BASE
+// for the digestion.  The entries are filled by one thread (add_load) before
+// the tasks are planned, by several: looking the kernels up for every task
+// behind their locks took 8 of 17 ms for the 23100 tasks of 100 waters.
 #define BQC_STEP_BASE 2
+struct ClassEntry {
+    bool filled = false;
+    RowKernel row = nullptr, wave[2] = {nullptr, nullptr};
+    unsigned row_waves = 0, wave_waves[2] = {0, 0};
+    double cost[2] = {0, 0};
+};
 struct ClassLoad {
-    double cost[2][BQC_NPAIRID][BQC_NPAIRID];
-    ClassLoad() { memset(cost, 0, sizeof(cost)); }
-    double &at(const TaskCtx &c, int prec) {
-        return c.swap ? cost[prec][c.pkl][c.pij] : cost[prec][c.pij][c.pkl];
+    ClassEntry entry[BQC_NPAIRID][BQC_NPAIRID];
+    // (tasks of the run-time-class kernel have no entry and read none)
+    ClassEntry &at(const TaskCtx &c) {
+        return c.gen ? entry[0][0] : (c.swap ? entry[c.pkl][c.pij] : entry[c.pij][c.pkl]);
     }
 };
+
+static void fill_entry(ClassEntry &e, const TaskCtx &c) {
+    if (e.filled) return;
+    e.filled = true;
+    auto usable = [&](const auto &t) {
+        const RowKernel r = c.swap ? t[c.pkl][c.pij] : t[c.pij][c.pkl];
+        return r && scratch_ok((const void *)r) ? r : nullptr;
+    };
+    e.row = usable(g_rows[0]);
+    if (e.row) e.row_waves = 4 * resident_blocks((const void *)e.row, 256);
+    for (int prec = 0; prec < 2; ++prec) {
+        e.wave[prec] = usable(g_waves[prec]);
+        if (e.wave[prec]) e.wave_waves[prec] = resident_blocks((const void *)e.wave[prec], 64);
+    }
+}
+
+// Kernels of a task per precision: the tile kernel of the class when there is
+// one, else the wave kernels.  False if there is neither (the generic kernels
+// take the task).  *log_cut: the precision rule, with every quartet in FP64
+// where the class has a tile kernel or no FP32 instance (FP64 code for k[1]
+// then, with no items).
+static bool pick_kernels(const TaskCtx &c, const ClassEntry &e, RowKernel (&k)[2], int (&wv)[2],
+                         double *log_cut) {
+    *log_cut = c.log_cut;
+    wv[0] = wv[1] = !e.row;
+    k[0] = e.row ? e.row : e.wave[0];
+    if (!k[0]) return false;
+    k[1] = e.row ? nullptr : e.wave[1];
+    if (!k[1]) {
+        k[1] = k[0];
+        *log_cut = -1e300;
+    }
+    return true;
+}
 
 static int step_cost(const TaskCtx &c) {
     return c.bp->cptype[c.cp_ij].nprim_12 * c.bp->cptype[c.cp_kl].nprim_12 + BQC_STEP_BASE;
@@ -669,7 +687,10 @@ static void add_load(ClassLoad &load, const TaskCtx &c) {
     RowKernel k[2];
     int wv[2];
     double log_cut;
-    if (c.gen || !pick_kernels(c, k, wv, &log_cut)) return;
+    if (c.gen) return;
+    ClassEntry &e = load.at(c);
+    fill_entry(e, c);
+    if (!pick_kernels(c, e, k, wv, &log_cut)) return;
     const int *pbins = c.swap ? c.bins_kl : c.bins_ij, *qbins = c.swap ? c.bins_ij : c.bins_kl;
     const int cp_p = c.swap ? c.cp_kl : c.cp_ij, cp_q = c.swap ? c.cp_ij : c.cp_kl;
     double steps[2] = {0, 0};
@@ -681,8 +702,8 @@ static void add_load(ClassLoad &load, const TaskCtx &c) {
         steps[0] += (wv[0] ? np : np / 64.0) * qsplit;
         steps[1] += (wv[1] ? np : np / 64.0) * (qmax - qsplit);
     }
-    if (is_tile(k[0])) steps[0] *= tile_parts(eval_cls(c));
-    for (int prec = 0; prec < 2; ++prec) load.at(c, prec) += steps[prec] * step_cost(c);
+    if (e.row) steps[0] *= tile_parts(eval_cls(c));
+    for (int prec = 0; prec < 2; ++prec) e.cost[prec] += steps[prec] * step_cost(c);
 }
 
 // Q pairs per work item of a task: at most the class's tile.  A wavefront
@@ -705,7 +726,7 @@ static void add_load(ClassLoad &load, const TaskCtx &c) {
 #define BQC_FILL_LO 0.25
 #define BQC_ITEM_MIN 96
 // share: work of the launch relative to what load holds.
-static int item_tile(ClassLoad &load, const TaskCtx &c, RowKernel kern, int wave, int prec,
+static int item_tile(const ClassEntry &e, const TaskCtx &c, RowKernel kern, int wave, int prec,
                      int nao, double share = 1) {
     bool fixed;
     int cap = tile_for(wave ? 4 : 1, eval_cls(c), prec, nao, &fixed);
@@ -713,11 +734,12 @@ static int item_tile(ClassLoad &load, const TaskCtx &c, RowKernel kern, int wave
     // the tile kernels' set-up is longer than the row kernels' whose bands
     // these are: 32 / 64 / 128 / 256 / 512 took 89.0 / 79.8 / 76.9 / 76.1 / 76.7
     // ms on 64 waters cc-pVDZ, within 1 % elsewhere
-    if (is_tile(kern)) cap = BQC_TILE_ITEM;
-    const unsigned waves = wave ? resident_blocks((const void *)kern, 64)
-                                : 4 * resident_blocks((const void *)kern, 256);
+    if (kern == e.row) cap = BQC_TILE_ITEM;
+    const unsigned waves = wave ? e.wave_waves[kern == e.wave[1]]
+                                : (kern == e.row ? e.row_waves
+                                                 : 4 * resident_blocks((const void *)kern, 256));
     if (!waves) return cap;
-    const double per_wave = share * load.at(c, prec) / waves;
+    const double per_wave = share * e.cost[prec] / waves;
     const double cost = std::max(per_wave / BQC_FILL_HI,
                                  std::min(per_wave / BQC_FILL_LO, (double)BQC_ITEM_MIN));
     const double ck = cost / step_cost(c);
@@ -731,27 +753,26 @@ static int item_tile(ClassLoad &load, const TaskCtx &c, RowKernel kern, int wave
 // (dd|pp) with 46 took 1.46 ms in parts against 1.14, (dd|ds) with 38 1.32
 // against 0.70, (dp|dp) with 60 1.40 against 1.98.
 #define BQC_PARTS_MIN_LOAD (50 * (1 + BQC_STEP_BASE))
-static RowKernel small_parts_kernel(const TaskCtx &c, RowKernel tile, ClassLoad &load) {
-    if (!is_tile(tile) || tile_parts(eval_cls(c)) <= 2) return nullptr;
-    RowKernel w = c.swap ? g_waves[0][c.pkl][c.pij] : g_waves[0][c.pij][c.pkl];
-    const unsigned waves = 4 * resident_blocks((const void *)tile, 256);
-    if (!w || !scratch_ok((const void *)w) || load.at(c, 0) >= (double)BQC_PARTS_MIN_LOAD * waves)
+static RowKernel small_parts_kernel(const TaskCtx &c, const ClassEntry &e) {
+    if (!e.row || tile_parts(eval_cls(c)) <= 2 ||
+        e.cost[0] >= (double)BQC_PARTS_MIN_LOAD * e.row_waves)
         return nullptr;
-    return w;
+    return e.wave[0];
 }
 
-// Adds one task to the plan; load holds the work of the whole launch set.
+// Adds one task to the plan; e holds the work of its class in the whole launch
+// set.
 // Returns -1 if the generic kernels take the task.
 template <template <class> class V>
 static int plan_task(BuildPlanT<V> &bp_, const TaskCtx &c, const int *bra_order,
-                     const JKArgs &jk, const PairData &pd, ClassLoad &load) {
+                     const JKArgs &jk, const PairData &pd, const ClassEntry &e) {
     if (!bra_order || c.gen) return -1;
     RowKernel k[2];
     int wv[2];
     double log_cut;
-    if (!pick_kernels(c, k, wv, &log_cut)) return -1;
+    if (!pick_kernels(c, e, k, wv, &log_cut)) return -1;
     double share = 1;
-    if (RowKernel w = small_parts_kernel(c, k[0], load)) {
+    if (RowKernel w = small_parts_kernel(c, e)) {
         k[0] = k[1] = w;
         wv[0] = wv[1] = 1;
         share = 64.0 / tile_parts(eval_cls(c));
@@ -817,9 +838,9 @@ static int plan_task(BuildPlanT<V> &bp_, const TaskCtx &c, const int *bra_order,
     // -> 9.6 ms, (ps|ss) 17.2 -> 14.4, 12 molecules def2-SVP (ps|ss) 27.0 ->
     // 25.5; (ps|ps) loses 0.6 ms there and gains 0.7 here, (pp|ps) loses 0.8,
     // and short items only gather more (8 waters 2.6 -> 2.9 ms).
-    const bool blocks = is_tile(k[0]) && class_components(eval_cls(c)) <= 9 && !t_noalloc &&
+    const bool blocks = k[0] == e.row && class_components(eval_cls(c)) <= 9 && !t_noalloc &&
                         log_cut <= -1e299 && bp->bas_pair2shls &&
-                        item_tile(load, c, k[0], 0, 0, jk.nao) >= 32;
+                        item_tile(e, c, k[0], 0, 0, jk.nao) >= 32;
     bp_.tasks.push_back(td);
     bp_.bins_off.push_back(bp_.ints.size());
     bp_.ints.insert(bp_.ints.end(), pbins, pbins + nbins + 1);
@@ -856,9 +877,9 @@ static int plan_task(BuildPlanT<V> &bp_, const TaskCtx &c, const int *bra_order,
         qmax = qbins[nbins - s];
         qsplit = qbins[fp32_split(c, cp_p, cp_q, pbins, qbins, s, log_cut)];
     };
-    const int parts = is_tile(k[0]) ? tile_parts(cls) : 1;
+    const int parts = k[0] == e.row ? tile_parts(cls) : 1;
     for (int prec = 0; prec < 2; ++prec) {
-        const int ck = item_tile(load, c, k[prec], wv[prec], prec, jk.nao, prec ? 1 : share);
+        const int ck = item_tile(e, c, k[prec], wv[prec], prec, jk.nao, prec ? 1 : share);
         const int step = wv[prec] ? 1 : 64;
         V<int> &it = g[prec]->items;
         for (int p = 0; p < np; p += step) {
@@ -1318,14 +1339,17 @@ static int task_ctx(TaskCtx &c, const MolArgs &a, int t, int nbins, int precisio
 static int plan_refs(BuildPlan &plan, const MolArgs *m, const TaskRef *list, size_t n,
                      int nbins, int precision, double fp32_cut, ClassLoad &load,
                      std::vector<Deferred> *deferred) {
+    int im = -1;
+    PairData pd;
     for (size_t i = 0; i < n; ++i) {
         const MolArgs &a = m[list[i].im];
         TaskCtx c;
         int err = task_ctx(c, a, list[i].t, nbins, precision, fp32_cut);
         if (err) return err;
         JKArgs jk = {a.vj, a.vk, a.dm, a.nao, a.n_dm};
-        PairData pd = make_pair_data(a.bp);
-        err = plan_task(plan, c, a.bra_order, jk, pd, load);
+        if (list[i].im != im) pd = make_pair_data(a.bp);
+        im = list[i].im;
+        err = plan_task(plan, c, a.bra_order, jk, pd, load.at(c));
         if (err < 0) {
             deferred->push_back(Deferred{c, jk, pd});
             err = 0;
@@ -1335,19 +1359,14 @@ static int plan_refs(BuildPlan &plan, const MolArgs *m, const TaskRef *list, siz
     return 0;
 }
 
-// Plans tasks list[0, n), with several host threads when there are enough:
+// Plans tasks list[0, n) of a launch set with the given load, with several host
+// threads when there are enough:
 // blocks of tasks handed out in order are planned into plans of their own
 // and merged in block order (the same plan as one pass over the list).
 // Generic-kernel tasks are appended to deferred in list order.
 static int plan_list(BuildPlan &plan, const MolArgs *m, const TaskRef *list, size_t n,
-                     int nbins, int precision, double fp32_cut, std::vector<Deferred> &deferred) {
-    ClassLoad load;
-    for (size_t i = 0; i < n; ++i) {
-        TaskCtx c;
-        const int err = task_ctx(c, m[list[i].im], list[i].t, nbins, precision, fp32_cut);
-        if (err) return err;
-        add_load(load, c);
-    }
+                     int nbins, int precision, double fp32_cut, ClassLoad &load,
+                     std::vector<Deferred> &deferred) {
     const int nth = plan_threads(n);
     if (nth < 2) return plan_refs(plan, m, list, n, nbins, precision, fp32_cut, load, &deferred);
     const size_t bsz = std::max<size_t>(4, n / ((size_t)nth * 8));
@@ -1408,8 +1427,9 @@ static int build_by_class(const MolArgs *m, int nmol, int nbins, int precision, 
     int err = check_build_args(m, nmol, nbins, precision);
     if (err) return err;
     register_kernels();
-    std::vector<int> keys;
     std::vector<std::vector<TaskRef>> by_cls;
+    std::vector<short> at(1111 * BQC_LMAX_GEN + 1, -1);  // place of a class in by_cls
+    ClassLoad load;
     double work = 0;
     for (int im = 0; im < nmol; ++im)
         for (int t = 0; t < m[im].ntask; ++t) {
@@ -1417,11 +1437,10 @@ static int build_by_class(const MolArgs *m, int nmol, int nbins, int precision, 
             err = task_ctx(c, m[im], t, nbins, precision, fp32_cut);
             if (err) return err;
             work += task_flops(c);
-            const int key = eval_cls(c);
-            size_t k = 0;
-            while (k < keys.size() && keys[k] != key) ++k;
-            if (k == keys.size()) {
-                keys.push_back(key);
+            add_load(load, c);
+            short &k = at[eval_cls(c)];
+            if (k < 0) {
+                k = (short)by_cls.size();
                 by_cls.emplace_back();
             }
             by_cls[k].push_back(TaskRef{im, t});
@@ -1444,7 +1463,7 @@ static int build_by_class(const MolArgs *m, int nmol, int nbins, int precision, 
         BuildPlan plan;
         std::vector<Deferred> def;
         err = plan_list(plan, m, by_cls[k].data(), by_cls[k].size(), nbins, precision, fp32_cut,
-                        def);
+                        load, def);
         for (Deferred &d : def)
             if (!err) err = launch_quartets(d.c, d.jk, d.pd, stream, plan.flops);
         const int on = rotate ? side->least(queued) : 0;
@@ -1468,13 +1487,21 @@ static int plan_molecules(BuildPlanT<V> &plan, const MolArgs *m, int nmol, int n
     const int cerr = check_build_args(m, nmol, nbins, precision);
     if (cerr) return cerr;
     register_kernels();
+    ClassLoad load;
+    for (int im = 0; im < nmol; ++im)
+        for (int t = 0; t < m[im].ntask; ++t) {
+            TaskCtx c;
+            const int err = task_ctx(c, m[im], t, nbins, precision, fp32_cut);
+            if (err) return err;
+            add_load(load, c);
+        }
     if constexpr (std::is_same<BuildPlanT<V>, BuildPlan>::value) {
         std::vector<TaskRef> list;
         for (int im = 0; im < nmol; ++im)
             for (int t = 0; t < m[im].ntask; ++t) list.push_back(TaskRef{im, t});
         std::vector<Deferred> def;
         const int err = plan_list(plan, m, list.data(), list.size(), nbins, precision, fp32_cut,
-                                  def);
+                                  load, def);
         if (err) return err;
         for (Deferred &d : def) {
             if (deferred) {
@@ -1486,14 +1513,6 @@ static int plan_molecules(BuildPlanT<V> &plan, const MolArgs *m, int nmol, int n
         }
         return 0;
     }
-    ClassLoad load;
-    for (int im = 0; im < nmol; ++im)
-        for (int t = 0; t < m[im].ntask; ++t) {
-            TaskCtx c;
-            const int err = task_ctx(c, m[im], t, nbins, precision, fp32_cut);
-            if (err) return err;
-            add_load(load, c);
-        }
     for (int im = 0; im < nmol; ++im) {
         const MolArgs &a = m[im];
         JKArgs jk = {a.vj, a.vk, a.dm, a.nao, a.n_dm};
@@ -1502,7 +1521,7 @@ static int plan_molecules(BuildPlanT<V> &plan, const MolArgs *m, int nmol, int n
             TaskCtx c;
             int err = task_ctx(c, a, t, nbins, precision, fp32_cut);
             if (err) return err;
-            err = plan_task(plan, c, a.bra_order, jk, pd, load);
+            err = plan_task(plan, c, a.bra_order, jk, pd, load.at(c));
             if (err < 0 && deferred) {
                 deferred->push_back(Deferred{c, jk, pd});
                 err = 0;
@@ -1602,7 +1621,7 @@ int GINTbuild_jk(BasisProdCache *bpcache, double *vj, double *vk, double *dm, in
     BuildPlan plan;
     ClassLoad load;
     add_load(load, c);
-    err = plan_task(plan, c, order, jk, pd, load);
+    err = plan_task(plan, c, order, jk, pd, load.at(c));
     if (err < 0) err = launch_quartets(c, jk, pd, stream, plan.flops);
     else if (err == 0) err = stage_and_launch(plan, stage_for(stream), stream);
     g_last_flops[0] = plan.flops[0];
