@@ -132,6 +132,9 @@ __device__ __forceinline__ void atomic_add(gdouble *p, double v) {
 // parallel chains; of which 5 ms go into rounding them like quotients).  The
 // P pairs of a wavefront's lanes lie apart: their records take 64 lines of L1
 // per primitive instead of 320 (181 -> 175 ms, 40 waters mixed 52.5 -> 50.1).
+// Both only where a wavefront shares its Q pair (ROW): elsewhere the registers
+// are full, and the four-index fill of 1 water cc-pVTZ took 65 ms with them, 52
+// without.
 // FLAT: all loops unrolled (needs a compile-time x0), so that the block stays
 // in registers.
 template <int LA, int LB, int LC, int LD, typename T, int XN = Cls<LA, LB, LC, LD>::NFI,
@@ -146,6 +149,7 @@ __device__ __forceinline__ void eri_block(T *__restrict__ gout, const PairData &
     constexpr int NR = C::NR;
     constexpr int NG = XN * C::NFJ * C::NFK * C::NFL;
     constexpr int UO = FLAT ? 16 : 1, UN = FLAT ? 2048 : 8;
+    constexpr bool ROW = !std::is_same<RysPtr, std::nullptr_t>::value;
 #pragma unroll UN
     for (int n = 0; n < NG; ++n) gout[n] = (T)0;
     const double ab[3] = {ra[0] - rb[0], ra[1] - rb[1], ra[2] - rb[2]};
@@ -168,7 +172,7 @@ __device__ __forceinline__ void eri_block(T *__restrict__ gout, const PairData &
             P[0] = p_first[2];
             P[1] = p_first[3];
             P[2] = p_first[4];
-        } else if (pd.prec) {
+        } else if (ROW && pd.prec) {
             const gptr<double> r = glb(pd.prec) + (size_t)p * BQC_PREC;
             aij = r[0];
             eij = r[1];
@@ -183,16 +187,36 @@ __device__ __forceinline__ void eri_block(T *__restrict__ gout, const PairData &
             P[2] = pz12[p];
         }
         // the next Q primitive pair is loaded while this one is used
-        double nakl = qa12[qq0], nekl = qe12[qq0], nQ[3] = {qx12[qq0], qy12[qq0], qz12[qq0]};
+        double nakl, nekl, nQ[3];
+        if constexpr (ROW) {
+            nakl = qa12[qq0];
+            nekl = qe12[qq0];
+            nQ[0] = qx12[qq0];
+            nQ[1] = qy12[qq0];
+            nQ[2] = qz12[qq0];
+        }
         for (int iq = 0; iq < np_q; ++iq) {
-            const double akl = nakl, ekl = nekl;
-            const double Q[3] = {nQ[0], nQ[1], nQ[2]};
-            const int qn = qq0 + (iq + 1 < np_q ? iq + 1 : iq);
-            nakl = qa12[qn];
-            nekl = qe12[qn];
-            nQ[0] = qx12[qn];
-            nQ[1] = qy12[qn];
-            nQ[2] = qz12[qn];
+            const int q = qq0 + iq;
+            double akl, ekl, Q[3];
+            if constexpr (ROW) {
+                akl = nakl;
+                ekl = nekl;
+                Q[0] = nQ[0];
+                Q[1] = nQ[1];
+                Q[2] = nQ[2];
+                const int qn = iq + 1 < np_q ? q + 1 : q;
+                nakl = qa12[qn];
+                nekl = qe12[qn];
+                nQ[0] = qx12[qn];
+                nQ[1] = qy12[qn];
+                nQ[2] = qz12[qn];
+            } else {
+                akl = qa12[q];
+                ekl = qe12[q];
+                Q[0] = qx12[q];
+                Q[1] = qy12[q];
+                Q[2] = qz12[q];
+            }
             const double pq[3] = {P[0] - Q[0], P[1] - Q[1], P[2] - Q[2]};
             const double aijkl = aij + akl;
             const double a1 = aij * akl;
@@ -248,12 +272,18 @@ __device__ __forceinline__ void eri_block(T *__restrict__ gout, const PairData &
             // after the work, so single-primitive pairs never wait on it).
             // Not in blocks above 81 components, whose registers are
             // full: there the test added spills ((dp|ds) 240 -> 268 ms).
-            if constexpr (NG <= 81)
-                if (nekl == 0.0) break;
+            if constexpr (NG <= 81) {
+                if constexpr (ROW) {
+                    if (nekl == 0.0) break;
+                } else {
+                    if (iq + 1 < np_q && qe12[q + 1] == 0.0) break;
+                }
+            }
         }
         if constexpr (NG <= 81)
             if (ip + 1 < np_p &&
-                (pd.prec ? glb(pd.prec)[(size_t)(p + 1) * BQC_PREC + 1] : pe12[p + 1]) == 0.0)
+                (ROW && pd.prec ? glb(pd.prec)[(size_t)(p + 1) * BQC_PREC + 1] : pe12[p + 1]) ==
+                    0.0)
                 break;
     }
 }
