@@ -1112,19 +1112,16 @@ static int launch_groups(const BuildPlanT<V> &p, const StagedT<V> &st, char *dev
             if (launch_group(p, st, dev, gi, stream)) return 1;
         return 0;
     }
-    // longest first, each to the stream with the least queued so far
-    std::vector<std::pair<double, size_t>> order(ng);
-    for (size_t gi = 0; gi < ng; ++gi)
-        order[gi] = {-(10 + 0.1 * class_components(p.groups[gi].cls) + p.groups[gi].flops / 4e6),
-                     gi};
-    std::sort(order.begin(), order.end());
-    double queued[BQC_SIDE_STREAMS + 1] = {};
+    // in plan order, the streams in turn.  By estimated time, longest first and
+    // each to the stream with the least queued, was slower (ms): 8 waters
+    // cc-pVDZ 1.66 against 1.55, 13 waters with two densities 5.05 / 4.71, 24
+    // molecules replayed 61.1 / 59.8; by FLOPs alone 1.73 / 1.70, 5.58 / 5.24,
+    // 60.9 / 60.7 (another card).
     if (side->begin(stream)) return 1;
     int err = 0;
-    for (const auto &o : order) {
-        const int k = side->least(queued);
-        queued[k] -= o.first;
-        err |= launch_group(p, st, dev, o.second, k ? side->s[k - 1] : stream);
+    for (size_t gi = 0; gi < ng; ++gi) {
+        const size_t k = gi % (BQC_SIDE_STREAMS + 1);
+        err |= launch_group(p, st, dev, gi, k ? side->s[k - 1] : stream);
     }
     return side->end(stream) ? 1 : err;
 }
