@@ -160,7 +160,6 @@ struct Cls {
     // outer loops (the block then lives in scratch memory)
     static constexpr bool BIG = NF > 160;
     static constexpr int UO = BIG ? 1 : 16;
-    static constexpr int UN = BIG ? 8 : 2048;
     __host__ __device__ static constexpr int g(int i, int j, int k, int l) {
         return i * S_I + j * S_J + k * S_K + l;
     }

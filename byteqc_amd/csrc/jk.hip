@@ -428,13 +428,15 @@ static int g_ck_rows = BQC_CK_ROWS_DEFAULT;  // Q pairs per row-kernel item
 static int g_ck_wave = BQC_CK_WAVE_DEFAULT;  // Q pairs per wave-kernel item
 static std::vector<std::pair<long long, int>> g_ck_override;  // (key, ck)
 
-// Default tiles by molecule size.  Autotuner timings on MI355X: for large
-// molecules (64 H2O cc-pVDZ, 2624 Cartesian AOs; 128 H2O cc-pVTZ) the row
-// kernels of the s/p classes are fastest with 256 Q pairs per item (fewer
-// flushes of the lane accumulators; 4-6 % over 64), the spilling 108-component
-// classes with 32-64 and the wave kernels with 64; for batches of small
-// molecules (4-40 H2O def2-SVP, at most ~1000 AOs) with 32, 16 and 16.
-// Launches with little work use shorter items (item_tile).
+// Size bands, as BQCget_tile reports them.  Autotuner timings on MI355X: for
+// large molecules (64 H2O cc-pVDZ, 2624 Cartesian AOs; 128 H2O cc-pVTZ) the
+// two-pass row kernels of the s/p classes are fastest with 256 Q pairs per item
+// (fewer flushes of the lane accumulators; 4-6 % over 64) and the wave kernels
+// with 64; for batches of small molecules (4-40 H2O def2-SVP, at most ~1000
+// AOs) the wave kernels with 16.  They cap the items of those kernels, which
+// launches with little work shorten; tile kernels have a cap of their own
+// (item_tile), so that no launch is cut by the row values of the smallest band
+// and of the classes above 81 components.
 #define BQC_TILE_BIG_NAO 2048
 #define BQC_TILE_HUGE_NAO 8192
 static bool g_ck_all_set[2] = {false, false};  // a tile set for all classes of a kind
@@ -451,12 +453,7 @@ static int tile_for(int kind, int cls, int prec, int nao, bool *fixed = nullptr)
         if (kv.first == key) return kv.second;
     if (g_ck_all_set[kind == 1 ? 0 : 1]) return kind == 1 ? g_ck_rows : g_ck_wave;
     if (fixed) *fixed = false;
-    // three size bands, read off the autotuner on MI355X (batches of 4-40
-    // waters, 64 waters cc-pVDZ, 128 waters cc-pVTZ): longer Q ranges per
-    // item pay as the molecule grows
-    // (batches of small molecules with persistent grids: longer ranges than
-    // mid-size molecules, except (ss|ss) and (pp|pp): 256 molecules of 4-40
-    // waters def2-SVP 4.65 -> 4.52 s per batch)
+    // longer Q ranges per item pay as the molecule grows
     const int band = nao >= BQC_TILE_HUGE_NAO ? 2 : (nao >= BQC_TILE_BIG_NAO ? 1 : 0);
     static const int wave[3] = {32, 32, 64}, rows_big[3] = {128, 64, 128},
                      rows[3] = {128, 64, 256};

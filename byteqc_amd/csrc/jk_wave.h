@@ -78,7 +78,9 @@ __device__ __forceinline__ int gidx(int n, int d) {
 // classes listed here that cost resident waves and made the kernel slower on
 // MI355X ((fd|dp) 106 -> 144 ms, (fp|pp) 153 -> 170 ms), so they load late.
 // Elsewhere early loads gain up to 25 % ((dp|dp) 412 -> 328 ms; measured per
-// class on 128 H2O cc-pVTZ with every class early and every class late).
+// class on 128 H2O cc-pVTZ with every class early and every class late).  Of the
+// classes listed, (dd|pp) and (fp|pp) run here only in small launches by now,
+// at which they were not timed again.
 template <int LA, int LB, int LC, int LD>
 constexpr bool wave_prefetch() {
     constexpr int c = LA * 1000 + LB * 100 + LC * 10 + LD;
@@ -90,7 +92,8 @@ constexpr bool wave_prefetch() {
 // budget the compiler picks by itself; for others it runs up to 3x slower
 // ((dd|dp) 40 -> 128 ms), and for (dp|pp) and (fp|ds) it no longer pays
 // (measured per class on 128 H2O cc-pVTZ with every wave class hinted and
-// with none), so the hint is per class.
+// with none), so the hint is per class.  (dd|ds), (fs|dp) and (fd|ps) run here
+// only in small launches by now, at which they were not timed again.
 template <int LA, int LB, int LC, int LD>
 constexpr int wave_min_waves() {
     constexpr int c = LA * 1000 + LB * 100 + LC * 10 + LD;
@@ -436,10 +439,13 @@ typedef WaveKernel WaveKernelTable[2][BQC_NPAIRID][BQC_NPAIRID];
 // quartets are few, so the alternative of one lane per quartet left the chip
 // empty behind single lanes of 10 000 components: 30 quartets of 5 waters
 // cc-pVTZ took 11.4 ms (0.3 ms here), 660 of 24 waters 25.8 ms (1.6 ms).
+// Tile classes in up to two parts never come here: only those of five and six
+// leave small launches to this kernel (small_parts_kernel).
 template <int LA, int LB, int LC, int LD>
 constexpr bool use_wave() {
     using C = Cls<LA, LB, LC, LD>;
-    return C::NF > 81 && (3 * C::NR * C::GSZ + C::NF) * 8 <= 130000;
+    return C::NF > 81 && (3 * C::NR * C::GSZ + C::NF) * 8 <= 130000 &&
+           !(use_tile<LA, LB, LC, LD>() && tile_parts<LA, LB, LC, LD>() <= 2);
 }
 
 template <int LA, int LB, int LC, int LD>
