@@ -48,3 +48,24 @@ def test_f_shells_take_turns():
         blocks[i, :, i] = 0
     assert not blocks.any()
     assert abs(k[::gold.K_STEP] - want['far_k']).max() < TOL and abs(k - k.T).max() < TOL
+
+
+# with the bound out of the way a mixed build runs exactly the classes without
+# a tile kernel in FP32 (test_jk_gpu.py compares such a build with FP64)
+def test_fp32_classes_of_cc_pvtz():
+    from byteqc_amd import systems
+    from byteqc_amd.scf import hf
+    mol = systems.water_mole(1, 4.0, 3, 'cc-pvtz')
+    pairs = [(a, b) for a in range(4) for b in range(a + 1)]
+    nf = lambda l: (l + 1) * (l + 2) // 2  # noqa: E731
+    want = {a * 1000 + b * 100 + c * 10 + d for i, (a, b) in enumerate(pairs)
+            for c, d in pairs[:i + 1] if nf(a) * nf(b) * nf(c) * nf(d) > 81} - PARTS
+    hf.profile_enable(True)
+    try:
+        hf.get_jk(mol, systems.random_density(mol.nao_nr(), 5, 2), precision='mixed',
+                  fp32_cut=1e30)
+        recs = [r for r in hf.profile_read() if r['nquart'] > 0]
+    finally:
+        hf.profile_enable(False)
+    assert {r['cls'] for r in recs if r['kind'] & 2} == want
+    assert {r['cls'] for r in recs if not r['kind'] & 2} >= PARTS
