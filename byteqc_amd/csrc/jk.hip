@@ -713,7 +713,17 @@ static void add_load(ClassLoad &load, const TaskCtx &c) {
 // more than BQC_FILL_LO items per resident wavefront allow.  Measured on
 // MI355X against fixed tiles (ms): 1 water cc-pVDZ 7.5 -> 1.2, 8 waters
 // cc-pVDZ 16.8 -> 4.1, 40 waters def2-SVP mixed 204 -> 68, 5 waters cc-pVTZ
-// 63.6 -> 27.  BQC_FILL_HI 4 / 8 / 16: 266 / 255 / 251 for 12 molecules
+// 63.6 -> 27.  Items of the row kernels cost at least BQC_ITEM_FLOOR (four
+// uncontracted steps) whatever the load: every item adds its J(a,b) to memory,
+// and a small molecule's (dd|ss) added 142 small terms one by one to sums
+// already complete, each rounded to their last place.  Error of J of 1 water
+// cc-pVDZ (cc-pVTZ), root mean square over the largest element, in 1e-17: 4.9
+// (7.2) without the floor and 12 (13) where those launches came last, 4.5 (6.0)
+// with it, 4.6 (6.1) with items of 128 pairs.  Without it / 12 / 24 (ms): 2
+// waters cc-pVDZ 0.63 / 0.57 / 0.66, 4 waters 1.08 / 0.86 / 0.84, 8 waters 1.82 /
+// 1.63 / 1.57, 2 waters cc-pVTZ 2.24 / 1.75 / 1.67, 1 water 0.51 / 0.53 / 0.62;
+// with the wave kernels under it too 2 waters cc-pVTZ 1.95.
+// BQC_FILL_HI 4 / 8 / 16: 266 / 255 / 251 for 12 molecules
 // def2-SVP, 200 / 201 / 205 for 24 waters cc-pVTZ; BQC_FILL_LO 0.06 / 0.25 /
 // 0.5: 32.8 / 27.0 / 26.7 for 5 waters cc-pVTZ, 4.6 / 4.1 / 4.8 for 8 waters
 // cc-pVDZ; BQC_ITEM_MIN 24 / 48 / 96 / 192: 12.6 / 11.8 / 11.8 / 13.8 for 13
@@ -722,6 +732,7 @@ static void add_load(ClassLoad &load, const TaskCtx &c) {
 #define BQC_FILL_HI 8
 #define BQC_FILL_LO 0.25
 #define BQC_ITEM_MIN 96
+#define BQC_ITEM_FLOOR 12
 // share: work of the launch relative to what load holds.
 static int item_tile(const ClassEntry &e, const TaskCtx &c, RowKernel kern, int wave, int prec,
                      int nao, double share = 1) {
@@ -737,8 +748,9 @@ static int item_tile(const ClassEntry &e, const TaskCtx &c, RowKernel kern, int 
                                                  : 4 * resident_blocks((const void *)kern, 256));
     if (!waves) return cap;
     const double per_wave = share * e.cost[prec] / waves;
-    const double cost = std::max(per_wave / BQC_FILL_HI,
-                                 std::min(per_wave / BQC_FILL_LO, (double)BQC_ITEM_MIN));
+    const double cost = std::max({per_wave / BQC_FILL_HI,
+                                  std::min(per_wave / BQC_FILL_LO, (double)BQC_ITEM_MIN),
+                                  wave ? 0.0 : (double)BQC_ITEM_FLOOR});
     const double ck = cost / step_cost(c);
     return ck >= cap ? cap : (ck > 1 ? (int)ck : 1);
 }
