@@ -1121,11 +1121,12 @@ static int launch_groups(const BuildPlanT<V> &p, const StagedT<V> &st, char *dev
             if (launch_group(p, st, dev, gi, stream)) return 1;
         return 0;
     }
-    // in plan order, the streams in turn.  By estimated time, longest first and
-    // each to the stream with the least queued, was slower (ms): 8 waters
-    // cc-pVDZ 1.66 against 1.55, 13 waters with two densities 5.05 / 4.71, 24
-    // molecules replayed 61.1 / 59.8; by FLOPs alone 1.73 / 1.70, 5.58 / 5.24,
-    // 60.9 / 60.7 (another card).
+    // in plan order, the streams in turn.  In turn / by estimated time, longest
+    // first and each to the stream with the least queued / in turn from the last
+    // class to the first (ms): 8 waters cc-pVDZ 1.63 / 1.66 / 1.58, 13 waters with
+    // two densities 5.22 / 5.67 / 5.15, 2 waters def2-SVP 1.60 / 1.91 / 1.58, 24
+    // molecules replayed 62.8 / 64.4 / 60.3, 4 of 2-6 waters replayed 1.60 / 1.59 /
+    // 1.71, 1 water cc-pVTZ 1.29 / 1.16 / 1.29, 2 waters 1.74 / 1.60 / 1.70.
     if (side->begin(stream)) return 1;
     int err = 0;
     for (size_t gi = 0; gi < ng; ++gi) {

@@ -1,5 +1,5 @@
 // Row kernel with its exchange block in LDS: the FP64 kernel of the classes up
-// to 81 components and of some up to 324, those in parts (tile_parts).
+// to 324 components except (ff|ps), the larger ones in parts (tile_parts).
 //
 // As in jk_rows a wavefront owns 64 pairs (a b) of the P list and walks a
 // range of the Q list in lock-step, and the six digestion sums are the same.
